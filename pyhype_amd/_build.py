@@ -9,6 +9,8 @@ from __future__ import annotations
 
 import os
 import subprocess
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
@@ -32,22 +34,35 @@ HIP_FLAGS = [
     "-Wno-unused-function",
 ]
 
-SOURCES = ["phx_kernels.hip", "phx_adjoint.hip"]
+# the stage kernels' instances are spread over several units: each takes minutes, and they compile in
+# parallel
+SOURCES = ["phx_stage_fused.hip", "phx_stage_lin.hip", "phx_stage_recon.hip", "phx_stage_yface.hip",
+           "phx_stage_gauss.hip", "phx_stage_shared.hip", "phx_adjoint.hip", "phx_kernels.hip"]
+
+
+def _run(cmd):
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"hipcc failed ({res.returncode}): {' '.join(cmd)}\n{res.stdout}\n{res.stderr}")
+    return res.stderr
 
 
 def build_library(verbose: bool = False, extra_flags=None) -> Path:
     """Compile every HIP source into ``lib/libpyhype_hip.so`` (always recompiles)."""
     LIBDIR.mkdir(exist_ok=True)
-    srcs = [str(CSRC / s) for s in SOURCES if (CSRC / s).exists()]
     tmp = LIB.with_suffix(".so.tmp")
-    cmd = [HIPCC, *HIP_FLAGS, *(extra_flags or []), "-shared", f"-I{INCLUDE}", *srcs, "-o", str(tmp)]
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    res = subprocess.run(cmd, capture_output=True, text=True)
-    if res.returncode != 0:
-        raise RuntimeError(f"hipcc failed ({res.returncode}):\n{res.stdout}\n{res.stderr}")
-    if verbose and res.stderr:
-        print(res.stderr)
+    jobs = max(1, min(len(SOURCES), int(os.environ.get("MAX_JOBS", 0)) or os.cpu_count() or 1, 8))
+    with tempfile.TemporaryDirectory(prefix="phx_build_") as tmpdir:
+        objs = [str(Path(tmpdir) / s.replace(".hip", ".o")) for s in SOURCES]
+        cmds = [[HIPCC, *HIP_FLAGS, *(extra_flags or []), f"-I{INCLUDE}", "-c", str(CSRC / s), "-o", o]
+                for s, o in zip(SOURCES, objs)]
+        if verbose:
+            print("\n".join(" ".join(c) for c in cmds), flush=True)
+        with ThreadPoolExecutor(jobs) as pool:
+            notes = list(pool.map(_run, cmds))
+        if verbose and any(notes):
+            print("".join(notes))
+        _run([HIPCC, f"--offload-arch={ARCH}", "-fPIC", "-shared", *objs, "-o", str(tmp)])
     os.replace(tmp, LIB)
     return LIB
 
@@ -60,9 +75,7 @@ def build_test_library(verbose: bool = False) -> Path:
     cmd = [HIPCC, *HIP_FLAGS, "-shared", f"-I{INCLUDE}", str(src), "-o", str(tmp)]
     if verbose:
         print(" ".join(cmd), flush=True)
-    res = subprocess.run(cmd, capture_output=True, text=True)
-    if res.returncode != 0:
-        raise RuntimeError(f"hipcc failed ({res.returncode}):\n{res.stdout}\n{res.stderr}")
+    _run(cmd)
     os.replace(tmp, out)
     return out
 

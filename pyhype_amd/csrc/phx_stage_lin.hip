@@ -1,0 +1,36 @@
+// phx_stage_lin.hip -- instances and launchers of the split stage's row-major reconstruction.
+#include "phx_stage.hpp"
+
+namespace phx {
+namespace stage {
+
+namespace {
+struct k_recon_x_lin_go {
+    template <bool C, int F, int M, bool G>
+    static void go(dim3 g, hipStream_t st, const StageArgs& A) {
+        constexpr int MM = G ? 3 : (M < 3 ? 3 : M);
+        hipLaunchKernelGGL((k_recon_x_lin<C ? 1 : 0, F, MM, G>), g, dim3(WAVE), 0, st, A);
+    }
+};
+}  // namespace
+
+void k_recon_x_lin_tag::launch(const phx_plan* P, int kind, int minw, dim3 g, hipStream_t st, const StageArgs& A) {
+    dispatch<k_recon_x_lin_go>(P, kind, minw, g, st, A);
+}
+
+// one launch of the reconstruction kernel of variant 7 over the merged list of both geometry kinds
+void launch_recon_x_lin_mixed(const phx_plan* P, StageArgs A, hipStream_t st) {
+    A.items = P->ditems_m[2];
+    A.nitems = P->n_m[2];
+    const dim3 g(P->grid_m[2]), b(WAVE);
+    const bool gen = generic_instance(P), roe = P->flux == PHX_FLUX_ROE;
+    const bool w4 = !gen && P->waves_per_simd >= 4;  // the register budgets the per-kind launches use
+#define PHX_RX(F, M, G) hipLaunchKernelGGL((k_recon_x_lin<2, F, M, G>), g, b, 0, st, A)
+    if (gen) { if (roe) PHX_RX(0, 3, true); else PHX_RX(1, 3, true); }
+    else if (w4) { if (roe) PHX_RX(0, 4, false); else PHX_RX(1, 4, false); }
+    else { if (roe) PHX_RX(0, 3, false); else PHX_RX(1, 3, false); }
+#undef PHX_RX
+}
+
+}  // namespace stage
+}  // namespace phx

@@ -1,0 +1,76 @@
+// phx_stage_shared.hip -- instances and launchers of the shared-halo, paired and element-wise stage kernels.
+#include "phx_stage.hpp"
+
+namespace phx {
+namespace stage {
+
+namespace {
+struct k_stage_wg_go {
+    template <bool C, int F, int M, bool G>
+    static void go(dim3 g, hipStream_t st, const StageArgs& A) {
+        hipLaunchKernelGGL((k_stage_wg<C, F, 2, G>), g, dim3(WGW * WAVE), 0, st, A);
+    }
+};
+struct k_stage_pair_go {
+    template <bool C, int F, int M, bool G>
+    static void go(dim3 g, hipStream_t st, const StageArgs& A) {
+        constexpr int MM = G ? 2 : (M > 3 ? 3 : (M < 2 ? 2 : M));
+        hipLaunchKernelGGL((k_stage_pair<C, F, MM, G>), g, dim3(PAIR_WAVES * WAVE), 0, st, A);
+    }
+};
+struct k_ew_recon_go {
+    template <bool C, int F, int M, bool G>
+    static void go(dim3 g, hipStream_t st, const StageArgs& A) {
+        hipLaunchKernelGGL((k_ew_recon<C ? 1 : 0, G>), g, dim3(EW_WG), 0, st, A);
+    }
+};
+struct k_ew_face_go {
+    template <bool C, int F, int M, bool G>
+    static void go(dim3 g, hipStream_t st, const StageArgs& A) {
+        hipLaunchKernelGGL((k_ew_face<C ? 1 : 0, F, G>), g, dim3(EW_WG), 0, st, A);
+    }
+};
+struct k_ew_update_go {
+    template <bool C, int F, int M, bool G>
+    static void go(dim3 g, hipStream_t st, const StageArgs& A) {
+        hipLaunchKernelGGL((k_ew_update<C ? 1 : 0>), g, dim3(EW_WG), 0, st, A);
+    }
+};
+}  // namespace
+
+void k_stage_wg_tag::launch(const phx_plan* P, int kind, int minw, dim3 g, hipStream_t st, const StageArgs& A) {
+    dispatch<k_stage_wg_go>(P, kind, minw, g, st, A);
+}
+void k_stage_pair_tag::launch(const phx_plan* P, int kind, int minw, dim3 g, hipStream_t st, const StageArgs& A) {
+    dispatch<k_stage_pair_go>(P, kind, minw, g, st, A);
+}
+void k_ew_recon_tag::launch(const phx_plan* P, int kind, int minw, dim3 g, hipStream_t st, const StageArgs& A) {
+    dispatch<k_ew_recon_go>(P, kind, minw, g, st, A);
+}
+void k_ew_face_tag::launch(const phx_plan* P, int kind, int minw, dim3 g, hipStream_t st, const StageArgs& A) {
+    dispatch<k_ew_face_go>(P, kind, minw, g, st, A);
+}
+void k_ew_update_tag::launch(const phx_plan* P, int kind, int minw, dim3 g, hipStream_t st, const StageArgs& A) {
+    dispatch<k_ew_update_go>(P, kind, minw, g, st, A);
+}
+
+void launch_ew_mixed(const phx_plan* P, StageArgs A, int p, hipStream_t st) {
+    A.items = P->ditems_em[p];
+    A.nitems = P->n_em[p];
+    const dim3 g(P->grid_em[p]), b(EW_WG);
+    const bool gen = generic_instance(P), roe = P->flux == PHX_FLUX_ROE;
+    if (p == 0) {
+        if (gen) hipLaunchKernelGGL((k_ew_recon<2, true>), g, b, 0, st, A);
+        else hipLaunchKernelGGL((k_ew_recon<2, false>), g, b, 0, st, A);
+    } else if (p == 1) {
+        if (roe && gen) hipLaunchKernelGGL((k_ew_face<2, 0, true>), g, b, 0, st, A);
+        else if (roe) hipLaunchKernelGGL((k_ew_face<2, 0, false>), g, b, 0, st, A);
+        else if (gen) hipLaunchKernelGGL((k_ew_face<2, 1, true>), g, b, 0, st, A);
+        else hipLaunchKernelGGL((k_ew_face<2, 1, false>), g, b, 0, st, A);
+    } else {
+        hipLaunchKernelGGL((k_ew_update<2>), g, b, 0, st, A);
+    }
+}
+
+}  // namespace stage
+}  // namespace phx
