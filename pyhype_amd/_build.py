@@ -36,8 +36,8 @@ HIP_FLAGS = [
 
 # the stage kernels' instances are spread over several units: each takes minutes, and they compile in
 # parallel
-SOURCES = ["phx_stage_fused.hip", "phx_stage_lin.hip", "phx_stage_recon.hip", "phx_stage_yface.hip",
-           "phx_stage_gauss.hip", "phx_stage_shared.hip", "phx_adjoint.hip", "phx_kernels.hip"]
+SOURCES = ["phx_stage_yface.hip", "phx_stage_fused.hip", "phx_stage_lin.hip", "phx_stage_recon.hip",
+           "phx_stage_shared.hip", "phx_adjoint.hip", "phx_kernels.hip"]
 
 
 def _run(cmd):
@@ -68,15 +68,16 @@ def build_library(verbose: bool = False, extra_flags=None) -> Path:
 
 
 def build_test_library(verbose: bool = False) -> Path:
-    """Compile the GPU tests' device numerics library (tests/native/libdevice_numerics.so)."""
-    src = PKG.parent / "tests" / "native" / "device_numerics.hip"
-    out = src.with_name("libdevice_numerics.so")
-    tmp = out.with_suffix(".so.tmp")
-    cmd = [HIPCC, *HIP_FLAGS, "-shared", f"-I{INCLUDE}", str(src), "-o", str(tmp)]
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    _run(cmd)
-    os.replace(tmp, out)
+    """Compile the tests' native libraries (tests/native/lib{device,inrange}_numerics.so)."""
+    native = PKG.parent / "tests" / "native"
+    for name in ("device_numerics", "inrange_numerics"):
+        out = native / f"lib{name}.so"
+        tmp = out.with_suffix(".so.tmp")
+        cmd = [HIPCC, *HIP_FLAGS, "-shared", f"-I{INCLUDE}", str(native / f"{name}.hip"), "-o", str(tmp)]
+        if verbose:
+            print(" ".join(cmd), flush=True)
+        _run(cmd)
+        os.replace(tmp, out)
     return out
 
 

@@ -234,12 +234,13 @@ __host__ __device__ inline Q4 cell_residual(const DevBlock& B, const AdjBlock& O
     for (int c = 0; c < 4; ++c) {
         if (nq > 1) {
             const double part = (LW * FW.v[c] - LE * FE.v[c]) + LS * FS.v[c];
-            R.v[c] = (0.5 * (part - LN * FN.v[c])) / A;
+            R.v[c] = 0.5 * (part - LN * FN.v[c]);
         } else {
             const double part = (LW * (2.0 * FW.v[c]) - LE * (2.0 * FE.v[c])) + LS * (2.0 * FS.v[c]);
-            R.v[c] = (0.5 * (part - LN * (2.0 * FN.v[c]))) / A;
+            R.v[c] = 0.5 * (part - LN * (2.0 * FN.v[c]));
         }
     }
+    phx::div_all(R.v, A, R.v);
     return R;
 }
 

@@ -28,6 +28,7 @@ struct DevBlock {
     const double* geom;
     const double* qoff;  // Gauss-point offsets (8*nq arrays of ny x nx) when nq > 1, else null
     double wall[8];
+    int odd;  // a geometry entry beyond 2^60 or an area below 2^-60 (CellGeo::odd)
 };
 
 // ---------------------------------------------------------------------------------------------
@@ -134,11 +135,12 @@ template <bool CG>
 __host__ __device__ inline phx::CellGeo cart_cell_geo(const DevBlock& B, const CartCols& c, int k, double Ac) {
     const CartGT<CG> G{B.geom, B.nx, B.ny};
     phx::CellGeo g;
+    g.odd = B.odd != 0;
     g.xlE = G.row(R_xlE, k); g.xlW = G.row(R_xlW, k);
     g.ylE = G.row(R_ylE, k); g.ylW = G.row(R_ylW, k);
     g.xlN = c.xlN; g.xlS = c.xlS;
     g.ylN = c.ylN; g.ylS = c.ylS;
-    g.ainv = 1.0 / Ac;
+    g.ainv = phx::inv_area(Ac);
     g.dxE = c.dxE; g.dxW = c.dxW;
     g.dxN = c.dxN; g.dxS = c.dxS;
     g.dyE = G.row(R_dyE, k); g.dyW = G.row(R_dyW, k);
@@ -276,13 +278,14 @@ __host__ __device__ inline phx::QGeo cell_qgeo(const DevBlock& B, int k, int j, 
 template <bool CART>
 __host__ __device__ inline phx::CellGeo cell_geo(const DevBlock& B, int k, int j) {
     phx::CellGeo g;
+    g.odd = B.odd != 0;
     if (CART) {
         const CartG G{B.geom, B.nx, B.ny};
         g.xlE = G.row(R_xlE, k); g.xlW = G.row(R_xlW, k);
         g.ylE = G.row(R_ylE, k); g.ylW = G.row(R_ylW, k);
         g.xlN = G.col(C_xlN, j); g.xlS = G.col(C_xlS, j);
         g.ylN = G.col(C_ylN, j); g.ylS = G.col(C_ylS, j);
-        g.ainv = 1.0 / G.A(k, j);
+        g.ainv = phx::inv_area(G.A(k, j));
         g.dxE = G.col(C_dxE, j); g.dxW = G.col(C_dxW, j);
         g.dxN = G.col(C_dxN, j); g.dxS = G.col(C_dxS, j);
         g.dyE = G.row(R_dyE, k); g.dyW = G.row(R_dyW, k);
@@ -293,7 +296,7 @@ __host__ __device__ inline phx::CellGeo cell_geo(const DevBlock& B, int k, int j
         g.ylE = G.V(F_yl, k, j + 1); g.ylW = -G.V(F_yl, k, j);
         g.xlN = G.H(F_xl, k + 1, j); g.xlS = -G.H(F_xl, k, j);
         g.ylN = G.H(F_yl, k + 1, j); g.ylS = -G.H(F_yl, k, j);
-        g.ainv = 1.0 / G.C(CL_A, k, j);
+        g.ainv = phx::inv_area(G.C(CL_A, k, j));
         const double xc = G.C(CL_xc, k, j), yc = G.C(CL_yc, k, j);
         g.dxE = G.V(F_xq, k, j + 1) - xc; g.dyE = G.V(F_yq, k, j + 1) - yc;
         g.dxW = G.V(F_xq, k, j) - xc; g.dyW = G.V(F_yq, k, j) - yc;

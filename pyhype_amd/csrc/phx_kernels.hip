@@ -28,8 +28,7 @@ int dt_slots_for(int ncases) {
 
 // standalone CFL reduction over the owned cells of every work item
 struct DtArgs {
-    const DevBlock* blocks;
-    const WorkItem* items;
+    const DevItem* items;
     int nitems;
     int strip;  // owned columns per item of this work list
     const double* U;
@@ -46,8 +45,8 @@ __global__ void __launch_bounds__(WAVE) k_dt(DtArgs A) {
     item_range(A.nitems, lo, hi, first, stride);
     const int lane = threadIdx.x & (WAVE - 1);
     for (int i = first; i < hi; i += stride) {
-        const WorkItem it = ld_const(A.items, i);
-        const DevBlock& B = A.blocks[it.block];
+        const DevItem& it = const_ref(A.items, i);
+        const DevBlock& B = it.b;
         const int j = it.j0 + lane;
         const bool own = (lane < A.strip) && (j < B.nx);
         double lane_dt = __longlong_as_double((long long)DT_INF_BITS);
@@ -206,16 +205,41 @@ int build_programs(phx_plan* P, int S, const double* a) {
     return PHX_OK;
 }
 
-int upload_items(std::vector<WorkItem> (&items)[2], WorkItem* (&ditems)[2], int (&grid)[2], int grid_waves) {
+// a work list on the device, each item with its block's descriptor
+int upload_list(const phx_plan* P, const std::vector<WorkItem>& items, DevItem*& dev) {
+    if (items.empty()) return PHX_OK;
+    std::vector<DevItem> full(items.size());
+    for (size_t i = 0; i < items.size(); ++i)
+        full[i] = DevItem{items[i].block, items[i].j0, items[i].r0, items[i].r1, P->hblocks[items[i].block]};
+    PHX_CK(hipMalloc(&dev, full.size() * sizeof(DevItem)));
+    PHX_CK(hipMemcpy(dev, full.data(), full.size() * sizeof(DevItem), hipMemcpyHostToDevice));
+    return PHX_OK;
+}
+
+int upload_items(const phx_plan* P, std::vector<WorkItem> (&items)[2], DevItem* (&ditems)[2], int (&grid)[2],
+                 int grid_waves) {
     for (int kind = 0; kind < 2; ++kind) {
         const size_t n = items[kind].size();
-        if (n) {
-            PHX_CK(hipMalloc(&ditems[kind], n * sizeof(WorkItem)));
-            PHX_CK(hipMemcpy(ditems[kind], items[kind].data(), n * sizeof(WorkItem), hipMemcpyHostToDevice));
-        }
+        const int rc = upload_list(P, items[kind], ditems[kind]);
+        if (rc) return rc;
         grid[kind] = (int)((grid_waves > 0 && (size_t)grid_waves < n) ? grid_waves : n);
     }
     return PHX_OK;
+}
+
+// Whether a block's geometry has an entry beyond 2^60 in magnitude (or not finite) or an area below
+// 2^-60: the range for which the limiter's in-range divisions are proven (limit_venkat).
+bool odd_geometry(const phx_block_desc& d) {
+    for (int64_t i = 0; i < d.geom_len; ++i)
+        if (!(fabs(d.geom[i]) <= 0x1p60)) return true;
+    const int64_t cells = (int64_t)d.nx * d.ny, V = (int64_t)d.ny * (d.nx + 1), H = (int64_t)(d.ny + 1) * d.nx;
+    const double* area = d.geom + (d.geom_kind == PHX_GEOM_CARTESIAN ? 8 + 11 * ((int64_t)d.nx + d.ny) : 7 * (V + H));
+    for (int64_t i = 0; i < cells; ++i)
+        if (!(area[i] >= 0x1p-60)) return true;
+    return false;
+}
+bool odd_gas(double gamma, double gm1) {
+    return !(gamma >= 0x1p-20 && gamma <= 0x1p20 && gm1 >= 0x1p-20 && gm1 <= 0x1p20);
 }
 
 // Work lists: per block, row ranges of `rows` rows times column strips.  The fused variant uses
@@ -377,26 +401,26 @@ int build_items(phx_plan* P) {
             deal_to_xcds(P->items_f[kind], P->xcd_chunk);
             for (int p = 0; p < 3; ++p) deal_to_xcds(P->items_e[p][kind], P->xcd_chunk);
         }
-    int rc = upload_items(P->items, P->ditems, P->grid, P->grid_waves);
+    int rc = upload_items(P, P->items, P->ditems, P->grid, P->grid_waves);
     if (rc) return rc;
-    rc = upload_items(P->items_b, P->ditems_b, P->grid_b, P->grid_waves);
+    rc = upload_items(P, P->items_b, P->ditems_b, P->grid_b, P->grid_waves);
     if (rc) return rc;
-    rc = upload_items(P->items_f, P->ditems_f, P->grid_f, P->grid_waves);
+    rc = upload_items(P, P->items_f, P->ditems_f, P->grid_f, P->grid_waves);
     if (rc) return rc;
     for (int p = 0; p < 3; ++p) {
-        rc = upload_items(P->items_e[p], P->ditems_e[p], P->grid_e[p], P->grid_waves);
+        rc = upload_items(P, P->items_e[p], P->ditems_e[p], P->grid_e[p], P->grid_waves);
         if (rc) return rc;
     }
     // both geometry kinds: one list per phase of the element-wise stage and of the split stages 6
     // and 7 with midpoint faces (one launch instead of two; the kernels choose the path per block)
-    auto merge = [&](const std::vector<WorkItem> (&two)[2], WorkItem*& dev, int& n_out, int& grid_out) -> int {
+    auto merge = [&](const std::vector<WorkItem> (&two)[2], DevItem*& dev, int& n_out, int& grid_out) -> int {
         if (two[0].empty() || two[1].empty()) return PHX_OK;
         std::vector<WorkItem> both(two[0]);
         both.insert(both.end(), two[1].begin(), two[1].end());
         if (P->grid_waves == 0) deal_to_xcds(both, P->xcd_chunk);
         const size_t n = both.size();
-        PHX_CK(hipMalloc(&dev, n * sizeof(WorkItem)));
-        PHX_CK(hipMemcpy(dev, both.data(), n * sizeof(WorkItem), hipMemcpyHostToDevice));
+        const int rc = upload_list(P, both, dev);
+        if (rc) return rc;
         n_out = (int)n;
         grid_out = (int)((P->grid_waves > 0 && (size_t)P->grid_waves < n) ? P->grid_waves : n);
         return PHX_OK;
@@ -442,7 +466,7 @@ StageArgs base_args(phx_plan* P) {
 // one launch of kernel family T over the items of one geometry kind; minw = register budget in
 // waves per SIMD (2, 3 or 4)
 template <class T>
-void launch_kind(const phx_plan* P, StageArgs A, int kind, const WorkItem* items, int nitems, int grid, int minw,
+void launch_kind(const phx_plan* P, StageArgs A, int kind, const DevItem* items, int nitems, int grid, int minw,
                  hipStream_t st) {
     A.items = items;
     A.nitems = nitems;
@@ -634,7 +658,7 @@ void launch_dt_reduce(phx_plan* P, const double* U, hipStream_t st) {
     for (int kind = 0; kind < 2; ++kind) {
         const int n = (int)P->items[kind].size();
         if (!n) continue;
-        DtArgs D{P->dblocks, P->ditems[kind], n, (P->variant == 1 || P->variant >= 5) ? STRIP_A : STRIP,
+        DtArgs D{P->ditems[kind], n, (P->variant == 1 || P->variant >= 5) ? STRIP_A : STRIP,
                  U, P->dtmin,
                  P->bad, P->step, P->nslot,
                  P->ph};
@@ -793,6 +817,7 @@ int phx_plan_create(const phx_plan_desc* D, phx_plan** out) {
     P->flux = D->flux;
     P->ph = Phys{D->gamma, D->gm1, D->one_over_gm1, D->g_over_gm1, D->cfl, D->limiter,
                  D->reconstruction == PHX_RECON_PRIMITIVE ? 1 : 0, nq};
+    P->ph.odd_gas = odd_gas(D->gamma, D->gm1) ? 1 : 0;
     P->desc.assign(D->blocks, D->blocks + D->nblocks);
     P->state_len = total;
     P->rows_per_item = D->rows_per_item > 0 ? D->rows_per_item : 32;
@@ -826,6 +851,7 @@ int phx_plan_create(const phx_plan_desc* D, phx_plan** out) {
         h.qoff = nq > 1 ? h.geom + (d.geom_len - 8LL * nq * d.nx * d.ny) : nullptr;
         if (d.geom_kind == PHX_GEOM_CARTESIAN)
             for (int q = 0; q < 8; ++q) h.wall[q] = d.geom[q];
+        h.odd = odd_geometry(d) ? 1 : 0;
         ghost_off[b] = gacc;
         gacc += 4LL * (2 * d.ny + 2 * d.nx);
     }

@@ -30,6 +30,7 @@ struct Phys {
     int limiter;  // PHX_LIMITER_* (0 = Venkatakrishnan)
     int prim;     // reconstruction in primitive variables (SolverConfig.reconstruction_type)
     int nq;       // Gauss points per face (SolverConfig.fvm_num_quadrature_points); 0 or 1: midpoint
+    int odd_gas;  // gamma or gamma - 1 outside [2^-20, 2^20]: the in-range divisions below are not used
 };
 
 template <class T>
@@ -38,19 +39,145 @@ struct PrimT {
 };
 using Prim = PrimT<double>;
 
+// Whether x holds on every / on any active lane of the wave (on the host: x).  A rare case is handled by
+// a branch of the whole wave, with the common path as the fall-through: on gfx950 a divergent `if`
+// costs about 30 cycles of a wave's time (the compare's round trip into the execution mask and back)
+// and a taken branch about 60 (14 with four waves on the SIMD), the price of 6 and 12 double
+// operations.  Both evaluations give the same bits, so a lane may take the general one without need.
+__host__ __device__ inline unsigned long long wave_lanes(bool x) {  // the lanes where x holds (host: 0 or 1)
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_ballot_w64(x);
+#else
+    return x ? 1ull : 0ull;
+#endif
+}
+__host__ __device__ inline bool wave_all(bool x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_ballot_w64(!x) == 0ull;
+#else
+    return x;
+#endif
+}
+__host__ __device__ inline bool wave_any(bool x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_ballot_w64(x) != 0ull;
+#else
+    return x;
+#endif
+}
+#define PHX_USUAL(x) __builtin_expect(!!(x), 1)
+#define PHX_RARE(x) __builtin_expect(!!(x), 0)
+
 __host__ __device__ inline Q4 q4zero() {
     Q4 q;
     q.v[0] = q.v[1] = q.v[2] = q.v[3] = 0.0;
     return q;
 }
 
+// IEEE division by a divisor whose magnitude, and that of the numerators, is known to be moderate.  The
+// compiler's sequence for n / d scales d and n where their exponents are extreme (v_div_scale), refines
+// v_rcp_f64 by two Newton steps, forms q = n*y, the remainder r = n - d*q and q + r*y (v_div_fmas,
+// which undoes the scaling), and replaces the result where an operand is zero, infinite or NaN or the
+// quotient is not a normal number (v_div_fixup).  For 2^-700 < |d| < 2^700 and |n / d| in
+// [2^-760, 2^760] with |n| > 2^-900 the scalings and that replacement are identities, so the
+// refinement alone gives the same bits: 8 instead of 11 instructions, no dependence on VCC between
+// two divisions, and one reciprocal for all numerators of a divisor (3 instructions each, 2 for 1/d).
+// A numerator of +-0 gives the zero of the right sign for d > 0 (the remainder is formed as d*q - n
+// so that -0 survives); for d < 0 the sign of a zero quotient is not defined.
+struct Recip {
+    double d;
+#if defined(__HIP_DEVICE_COMPILE__)
+    double y;
+#endif
+    __host__ __device__ explicit Recip(double x) : d(x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+        const double y0 = __builtin_amdgcn_rcp(x);
+        const double y1 = __builtin_fma(y0, __builtin_fma(-x, y0, 1.0), y0);
+        y = __builtin_fma(y1, __builtin_fma(-x, y1, 1.0), y1);
+#endif
+    }
+    __host__ __device__ double div(double n) const {
+#if defined(__HIP_DEVICE_COMPILE__)
+        const double q = n * y;
+        return __builtin_fma(-__builtin_fma(d, q, -n), y, q);
+#else
+        return n / d;
+#endif
+    }
+    __host__ __device__ double inv() const {
+#if defined(__HIP_DEVICE_COMPILE__)
+        return __builtin_fma(-__builtin_fma(d, y, -1.0), y, y);
+#else
+        return 1.0 / d;
+#endif
+    }
+};
+// The divisor of a function that is written once for both cases: FAST = true is a Recip (the caller
+// has established the ranges), FAST = false the plain division of any type.
+template <bool FAST, class T>
+struct Divisor {
+    T d;
+    __host__ __device__ explicit Divisor(const T& x) : d(x) {}
+    template <class N>
+    __host__ __device__ N div(const N& n) const { return n / d; }
+    __host__ __device__ T inv() const { return 1.0 / d; }
+};
+template <>
+struct Divisor<true, double> : Recip {
+    using Recip::Recip;
+};
+
+// x is 0 or |x| >= lo (false for NaN)
+__host__ __device__ inline int zero_or_from(double x, double lo) { return (fabs(x) >= lo) | (x == 0.0); }
+// x is 0 or 2^-600 <= |x| <= 2^600 (false for NaN)
+__host__ __device__ inline int moderate(double x) {
+    const double t = fabs(x);
+    return ((t >= 0x1p-600) & (t <= 0x1p600)) | (x == 0.0);
+}
+__host__ __device__ inline unsigned hi_word(double x) {
+    return (unsigned)(__builtin_bit_cast(unsigned long long, x) >> 32);
+}
+// all four of a, b, c, d are positive and in [2^-100, 2^100 (1 + 2^-20)]: the high words, which order
+// positive doubles, compared as unsigned integers (a negative value, an infinity or NaN is outside)
+__host__ __device__ inline int positive_moderate(double a, double b, double c, double d) {
+    const unsigned lo = 0x39b00000u, span = 0x46300000u - 0x39b00000u;  // high words of 2^-100 and 2^100
+    const unsigned x = hi_word(a) - lo, y = hi_word(b) - lo, z = hi_word(c) - lo, w = hi_word(d) - lo;
+    const unsigned m = x > y ? x : y, n = z > w ? z : w;
+    return (m > n ? m : n) <= span;
+}
+
+// q[c] = n[c] / d for N numerators (in place is fine): one reciprocal where d lies in [2^-100, 2^100] and
+// every numerator is 0 or moderate, plain divisions otherwise (a branch that waves without such a
+// lane skip).
+template <int N, class T>
+__host__ __device__ inline void div_all(const T (&n)[N], const T& d, T (&q)[N]) {
+    if constexpr (std::is_same<T, double>::value) {
+        int in = positive_moderate(d, d, d, d);
+#pragma unroll
+        for (int c = 0; c < N; ++c) in &= moderate(n[c]);
+        if (PHX_USUAL(wave_all(in))) {
+            const Recip by(d);
+#pragma unroll
+            for (int c = 0; c < N; ++c) q[c] = by.div(n[c]);
+            return;
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < N; ++c) q[c] = n[c] / d;
+}
+__host__ __device__ inline double inv_area(double A) {
+    if (PHX_USUAL(wave_all(positive_moderate(A, A, A, A)))) return Recip(A).inv();
+    return 1.0 / A;
+}
+
 // IEEE square root of a double.  The compiler's sequence scales x by 2^256 when x < 2^-767, runs
 // v_rsq_f64 and a Newton-Raphson refinement (g = x*y, h = y/2, r = 1/2 - h*g, g += g*r, h += h*r,
 // then twice g += (x - g*g)*h), scales back by 2^-128, and returns x itself for +-0 and +inf.  For
 // 2^-767 <= x <= DBL_MAX the scalings and that select are identities, so the refinement alone gives
-// the same bits: sqrt_rn evaluates it and takes the library sqrt only for other x (a branch that
-// waves skip when no lane needs it), 12 instead of 17 instructions with the range test.
-__host__ __device__ inline double sqrt_rn(double x) {
+// the same bits (sqrt_in_range, 10 instructions); sqrt_rn evaluates it and takes the library sqrt only
+// for other x (a branch that waves skip when no lane needs it), 12 instead of 17 instructions with
+// the range test.
+__host__ __device__ inline double sqrt_in_range(double x) {
 #if defined(__HIP_DEVICE_COMPILE__)
     const double y = __builtin_amdgcn_rsq(x);
     double g = x * y;
@@ -61,7 +188,14 @@ __host__ __device__ inline double sqrt_rn(double x) {
     h = __builtin_fma(h, r, h);
     g = __builtin_fma(d, h, g);
     d = __builtin_fma(-g, g, x);
-    g = __builtin_fma(d, h, g);
+    return __builtin_fma(d, h, g);
+#else
+    return sqrt(x);
+#endif
+}
+__host__ __device__ inline double sqrt_rn(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    double g = sqrt_in_range(x);
     if (!(x >= 0x1p-767 && x <= 0x1.fffffffffffffp+1023)) {
         // an empty volatile asm keeps this a branch: the compiler would otherwise evaluate the
         // library sqrt for every lane and select
@@ -74,25 +208,47 @@ __host__ __device__ inline double sqrt_rn(double x) {
     return sqrt(x);
 #endif
 }
-// sqrt of the flux arithmetic: sqrt_rn for doubles, the type's own sqrt otherwise
-template <class T>
+// sqrt of the flux arithmetic: sqrt_rn (FAST: sqrt_in_range) for doubles, the type's own sqrt otherwise
+template <bool FAST, class T>
 __host__ __device__ inline T sqrt_f(T x) {
-    return sqrt(x);
+    if constexpr (std::is_same<T, double>::value) return FAST ? sqrt_in_range(x) : sqrt_rn(x);
+    else return sqrt(x);
 }
-__host__ __device__ inline double sqrt_f(double x) { return sqrt_rn(x); }
 
 // ConservativeConverter.to_primitive (states/converter/concrete_defs.py:85-100), with
 // u = rhou/rho, v = rhov/rho (conservative.py:85-99), ek = rho*Ek, Ek = 0.5*(u*u+v*v)
 // (conservative.py:118-124), p = (gamma-1)*(e - ek) (conservative.py:107-110).
-template <class T>
-__host__ __device__ inline PrimT<T> cons_to_prim(const Q4T<T>& q, const Phys& ph) {
+template <bool FAST, class T>
+__host__ __device__ inline PrimT<T> cons_to_prim_f(const Q4T<T>& q, const Phys& ph) {
     PrimT<T> w;
+    const Divisor<FAST, T> by(q.v[0]);
     w.r = q.v[0];
-    w.u = q.v[1] / w.r;
-    w.v = q.v[2] / w.r;
+    w.u = by.div(q.v[1]);
+    w.v = by.div(q.v[2]);
     const T ek = w.r * (0.5 * (w.u * w.u + w.v * w.v));
     w.p = ph.gm1 * (q.v[3] - ek);
     return w;
+}
+template <class T>
+__host__ __device__ inline PrimT<T> cons_to_prim(const Q4T<T>& q, const Phys& ph) {
+    return cons_to_prim_f<false>(q, ph);
+}
+// The two states of a face: one reciprocal per state where, on the whole wave, both densities lie in
+// [2^-100, 2^100] and every momentum is 0 or moderate (the quotients then lie in [2^-701, 2^701]), plain
+// divisions otherwise.
+template <class T>
+__host__ __device__ inline void cons_to_prim2(const Q4T<T>& a, const Q4T<T>& b, const Phys& ph, PrimT<T>& L,
+                                              PrimT<T>& R) {
+    if constexpr (std::is_same<T, double>::value) {
+        if (PHX_USUAL(wave_all(positive_moderate(a.v[0], a.v[0], b.v[0], b.v[0]) & moderate(a.v[1]) & moderate(a.v[2]) &
+                               moderate(b.v[1]) & moderate(b.v[2])))) {
+            L = cons_to_prim_f<true>(a, ph);
+            R = cons_to_prim_f<true>(b, ph);
+            return;
+        }
+    }
+    L = cons_to_prim_f<false>(a, ph);
+    R = cons_to_prim_f<false>(b, ph);
 }
 
 // rotate_JIT / unrotate_JIT (utils/utils.py:75-85,148-158) with c = cos(theta), s = sin(theta).
@@ -141,8 +297,18 @@ __host__ __device__ inline void harten(T Rslow, T Rfast, T Lslow, T Lfast, T& l1
     T tm = 2.0 * (Rfast - Lfast);
     tp = (tp <= 0.0) ? T(1e-8) : tp;
     tm = (tm <= 0.0) ? T(1e-8) : tm;
-    if (fabs(l1) < tp) l1 = 0.5 * ((l1 * l1) / tp + tp);
-    if (fabs(l4) < tm) l4 = 0.5 * ((l4 * l4) / tm + tm);
+    if constexpr (std::is_same<T, double>::value) {
+        // few waves hold a face whose speed is that close to 0: the whole wave skips the divisions
+        const bool f1 = fabs(l1) < tp, f4 = fabs(l4) < tm;
+        if (PHX_RARE(wave_any(f1 | f4))) {
+            const double c1 = 0.5 * ((l1 * l1) / tp + tp), c4 = 0.5 * ((l4 * l4) / tm + tm);
+            l1 = f1 ? c1 : l1;
+            l4 = f4 ? c4 : l4;
+        }
+    } else {
+        if (fabs(l1) < tp) l1 = 0.5 * ((l1 * l1) / tp + tp);
+        if (fabs(l4) < tm) l4 = 0.5 * ((l4 * l4) / tm + tm);
+    }
 }
 
 // A face of a flat region: every jump dW = W_R - W_L is +0 (all bits zero), with a density and a
@@ -150,7 +316,8 @@ __host__ __device__ inline void harten(T Rslow, T Rfast, T Lslow, T Lfast, T& l1
 // dissipation below is finite and each term of Rc|Lambda|Lp dW is a finite number times +0, so the
 // four row sums are signed zeros: rows 0, 2 and 3 are +0 (each contains a term 1.0*z or Ek*z1 that
 // is +0), and row 1's sign does not matter because 0.5*(F_L1 + F_R1) >= p > 0.  The flux is then
-// exactly 0.5*(F_L + F_R), and roe_flux skips the square roots and divisions of the dissipation.
+// exactly 0.5*(F_L + F_R), and a wave whose faces are all flat skips the square roots and divisions of
+// the dissipation.
 __host__ __device__ inline bool roe_flat(double dr, double du, double dv, double dp, const PrimT<double>& L) {
     const unsigned long long z = __builtin_bit_cast(unsigned long long, dr) | __builtin_bit_cast(unsigned long long, du) |
                                  __builtin_bit_cast(unsigned long long, dv) | __builtin_bit_cast(unsigned long long, dp);
@@ -158,9 +325,53 @@ __host__ __device__ inline bool roe_flat(double dr, double du, double dv, double
     return z == 0ull && L.r >= lo && L.r <= hi && L.p >= lo && L.p <= hi && fabs(L.u) <= hi && fabs(L.v) <= hi;
 }
 
+// What the fluxes take from the two states by division and square root: the sqrt(rho)-weighted state
+// (RoePrimitiveState._roe_state_from_prim_JIT, states/primitive.py:301-320), the sound speeds of the
+// three states, h = gamma/(gamma-1) p*/rho* and 1/a* (ROE), and p/(gamma-1) of both states (HLLL).
+template <class T>
+struct RoeAvgT {
+    T r, u, v, p, aL, aR, a, h, ia, eL, eR;
+};
+// FAST: densities and pressures in [2^-100, 2^100] and a moderate gamma.  Every divisor is then moderate:
+// sqrt(rho_L) + sqrt(rho_R) in [2^-49, 2^52], the densities, rho* in [2^-100, 2^101], gamma - 1 and
+// a* = sqrt(gamma p*/rho*) in [2^-111, 2^111], and so is every numerator (1, p, gamma p,
+// (gamma/(gamma-1)) p*); the square roots' arguments lie in [2^-222, 2^222].
+template <bool FAST, bool HLLL, class T>
+__host__ __device__ inline void roe_avg_f(const PrimT<T>& L, const PrimT<T>& R, const Phys& ph, RoeAvgT<T>& m) {
+    const T sL = sqrt_f<FAST>(L.r), sR = sqrt_f<FAST>(R.r);
+    const T inv = Divisor<FAST, T>(sL + sR).inv();
+    m.r = sqrt_f<FAST>(L.r * R.r);
+    m.u = (L.u * sL + R.u * sR) * inv;
+    if (!HLLL) m.v = (L.v * sL + R.v * sR) * inv;
+    m.p = (L.p * sL + R.p * sR) * inv;
+    m.aL = sqrt_f<FAST>(Divisor<FAST, T>(L.r).div(ph.gamma * L.p));
+    m.aR = sqrt_f<FAST>(Divisor<FAST, T>(R.r).div(ph.gamma * R.p));
+    const Divisor<FAST, T> by_r(m.r);
+    m.a = sqrt_f<FAST>(by_r.div(ph.gamma * m.p));
+    if (HLLL) {
+        const Divisor<FAST, double> by_gm1(ph.gm1);
+        m.eL = by_gm1.div(L.p);
+        m.eR = by_gm1.div(R.p);
+    } else {
+        m.h = by_r.div(ph.g_over_gm1 * m.p);
+        m.ia = Divisor<FAST, T>(m.a).inv();
+    }
+}
+template <bool HLLL = false, class T>
+__host__ __device__ inline RoeAvgT<T> roe_avg(const PrimT<T>& L, const PrimT<T>& R, const Phys& ph) {
+    RoeAvgT<T> m;
+    if constexpr (std::is_same<T, double>::value) {
+        if (PHX_USUAL(!ph.odd_gas && wave_all(positive_moderate(L.r, R.r, L.p, R.p)))) {
+            roe_avg_f<true, HLLL>(L, R, ph, m);
+            return m;
+        }
+    }
+    roe_avg_f<false, HLLL>(L, R, ph, m);
+    return m;
+}
+
 // FluxRoe.compute_flux (flux/Roe.py:262-304) for one face, primitive left/right states.
-//  * Roe state: RoePrimitiveState._roe_state_from_prim_JIT (states/primitive.py:301-320) --
-//    note the sqrt(rho)-weighted pressure.
+//  * Roe state: roe_avg -- note the sqrt(rho)-weighted pressure.
 //  * F from primitives: PrimitiveState._F_from_prim_JIT (states/primitive.py:223-237).
 //  * Dissipation Rc |Lambda| Lp dW with the SciPy COO accumulation order of the reference's
 //    block layout (flux/eigen_system.py:115-158,205-242; values flux/Roe.py:175-260).  The
@@ -177,7 +388,7 @@ __host__ __device__ inline Q4T<T> roe_flux(const PrimT<T>& L, const PrimT<T>& R,
     if constexpr (std::is_same<T, double>::value) {
         // flat region: the dissipation is exactly zero (roe_flat); the derivative of the dissipation
         // is not, so the tangent-linear instantiation always evaluates it
-        if (roe_flat(R.r - L.r, R.u - L.u, R.v - L.v, R.p - L.p, L)) {
+        if (PHX_RARE(wave_all(roe_flat(R.r - L.r, R.u - L.u, R.v - L.v, R.p - L.p, L)))) {
             Q4T<T> F;
             F.v[0] = 0.5 * (FL0 + FR0);
             F.v[1] = 0.5 * (FL1 + FR1);
@@ -187,26 +398,18 @@ __host__ __device__ inline Q4T<T> roe_flux(const PrimT<T>& L, const PrimT<T>& R,
         }
     }
 
-    const T sL = sqrt_f(L.r), sR = sqrt_f(R.r);
-    const T inv = 1.0 / (sL + sR);
-    const T rs = sqrt_f(L.r * R.r);
-    const T us = (L.u * sL + R.u * sR) * inv;
-    const T vs = (L.v * sL + R.v * sR) * inv;
-    const T ps = (L.p * sL + R.p * sR) * inv;
-
-    const T aL = sqrt_f(ph.gamma * L.p / L.r);
-    const T aR = sqrt_f(ph.gamma * R.p / R.r);
-    const T as = sqrt_f(ph.gamma * ps / rs);
+    const RoeAvgT<T> m = roe_avg(L, R, ph);
+    const T us = m.u, vs = m.v, as = m.a, aL = m.aL, aR = m.aR;
     T l1 = us - as, l4 = us + as;
     harten(R.u - aR, R.u + aR, L.u - aL, L.u + aL, l1, l4);
 
     const T Ek = 0.5 * (us * us + vs * vs);           // Ek_JIT
-    const T H = ph.g_over_gm1 * ps / rs + Ek;         // H_given_Ek_JIT
+    const T H = m.h + Ek;                             // H_given_Ek_JIT
     const T ua = us * as;
-    const T ia = 1.0 / as;                            // compute_Lp
+    const T ia = m.ia;                                // compute_Lp
     const T ia2 = ia * ia;
     const T h = 0.5 * ia2;
-    const T r2a = 0.5 * rs * ia;
+    const T r2a = 0.5 * m.r * ia;
 
     const T d0 = R.r - L.r, d1 = R.u - L.u, d2 = R.v - L.v, d3 = R.p - L.p;
     // Lp * dW: rows in COO order (3,1),(1,0),(2,2),(3,3),(0,1),(1,3),(0,3)
@@ -523,14 +726,11 @@ __host__ __device__ inline bool nrm4_in_range(double x) {
     return t == 0.0 || (t >= 0x1p-400 && t <= 0x1p400);
 }
 
-// Euclidean norm of a 4-vector as dnrm2 computes it (see above).  Non-finite components take the
-// double formula (inf or NaN, as the extended computation gives).  Components within [2^-400, 2^400]
-// take the pair-of-doubles evaluation, which decides all but about one in 10^5 of them; the rest, and
-// components outside that range, take the integer emulation.  Force-inlined: the kernels make no
-// device-function calls.
-__host__ __device__ __forceinline__ double nrm4(double a, double b, double c, double d) {
-    // all components +-0 (the jumps across a face of a flat region): the extended sum is 0 and so
-    // is the norm; the emulation below is skipped by whole waves there
+// The norm where the pairs or the integers decide it: components of 0 or magnitude in [2^-400, 2^400] take
+// the pair-of-doubles evaluation, which decides all but about one in 10^5 of them; the rest, and components
+// outside that range, take the integer emulation; non-finite components the double formula (inf or
+// NaN, as the extended computation gives).
+__host__ __device__ __forceinline__ double nrm4_pairs(double a, double b, double c, double d) {
     if (((dbits(a) | dbits(b) | dbits(c) | dbits(d)) & 0x7fffffffffffffffull) == 0ull) return 0.0;
     const unsigned long long ex = 0x7ff0000000000000ull;
     if ((dbits(a) & ex) == ex || (dbits(b) & ex) == ex || (dbits(c) & ex) == ex || (dbits(d) & ex) == ex)
@@ -549,17 +749,57 @@ __host__ __device__ __forceinline__ double nrm4(double a, double b, double c, do
     return nrm4_ext(a, b, c, d);
 }
 
+// n / d to about 2^-46 of itself, for d in range
+__host__ __device__ inline double quotient_46(double n, double d) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const double y = __builtin_amdgcn_rcp(d);
+    return n * __builtin_fma(y, __builtin_fma(-d, y, 1.0), y);
+#else
+    return n / d;
+#endif
+}
+
+// Euclidean norm of a 4-vector as dnrm2 computes it (see above).  Force-inlined: the kernels make no
+// device-function calls.
+//
+// The extended computation rounds every square, sum and the root to 64 bits: its root is within
+// 3 * 2^-64 of itself of the exact one (squares and three sums 4 * 2^-64, halved by the root, whose own
+// rounding adds 2^-64).  So its rounding to double is that of the exact root wherever the exact root is
+// further from a midpoint of two doubles than that, at most 2^-8.4 of half a last place.  Here
+// the exact sum of squares is formed as a pair of doubles (to about 2^-100), y = RN(sqrt) of its high
+// part and the remainder delta = (S - y^2)/(2y), known to 2^-40 of itself, tell on which side of y's
+// midpoints the root lies; about one vector in 250 lies within 2^-8 of half a last place of one (or
+// y is a power of two, whose lower midpoint is nearer): a wave with such a lane, or with a sum outside
+// [2^-600, 2^1000], takes nrm4_pairs.  About 65 instead of 300 instructions, the same bits.
+__host__ __device__ __forceinline__ double nrm4(double a, double b, double c, double d) {
+    const bool zero = ((dbits(a) | dbits(b) | dbits(c) | dbits(d)) & 0x7fffffffffffffffull) == 0ull;
+    if (PHX_RARE(wave_all(zero))) return 0.0;  // the jumps across the faces of a flat region
+    const double pa = a * a, pb = b * b, pc = c * c, pd = d * d;
+    const double e = (fma(a, a, -pa) + fma(b, b, -pb)) + (fma(c, c, -pc) + fma(d, d, -pd));
+    const DD s1 = two_sum(pa, pb), s2 = two_sum(pc, pd), s3 = two_sum(s1.hi, s2.hi);
+    const double tail = (s1.lo + s2.lo) + (s3.lo + e);
+    const double S = s3.hi + tail;           // renormalised: |lo| <= half a last place of S,
+    const double lo = tail - (S - s3.hi);    // so the root lies within one last place of y
+    const unsigned hs = hi_word(S) - 0x1a700000u;  // high word of 2^-600
+    const bool in = hs <= 0x7e700000u - 0x1a700000u;
+    const double y = sqrt_in_range(S);
+    const double delta = quotient_46(fma(-y, y, S) + lo, 2.0 * y);  // S - y*y is exact
+    const unsigned long long yb = dbits(y);
+    // half of y's last place, and delta against it
+    const double half = __builtin_bit_cast(double, (yb & 0x7ff0000000000000ull) - (53ull << 52));
+    const double m = fabs(delta);
+    const bool sure = (fabs(m - half) > half * 0x1p-8) & ((yb & 0x000fffffffffffffull) != 0ull);
+    if (PHX_RARE(!wave_all(zero | (in & sure)))) return nrm4_pairs(a, b, c, d);
+    double r = y;
+    if (m > half) r = delta > 0.0 ? y + 2.0 * half : y - 2.0 * half;
+    return zero ? 0.0 : r;
+}
+
 // FluxHLLL.compute_flux + _HLLL_flux_JIT (flux/HLLL.py:25-49,70-103) for one face.
 template <class T>
 __host__ __device__ inline Q4T<T> hlll_flux(const PrimT<T>& L, const PrimT<T>& R, const Phys& ph) {
-    const T sL = sqrt_f(L.r), sR = sqrt_f(R.r);
-    const T inv = 1.0 / (sL + sR);
-    const T rs = sqrt_f(L.r * R.r);
-    const T us = (L.u * sL + R.u * sR) * inv;
-    const T ps = (L.p * sL + R.p * sR) * inv;
-    const T as = sqrt_f(ph.gamma * ps / rs);
-    const T aL = sqrt_f(ph.gamma * L.p / L.r);
-    const T aR = sqrt_f(ph.gamma * R.p / R.r);
+    const RoeAvgT<T> m = roe_avg<true>(L, R, ph);
+    const T us = m.u, as = m.a, aL = m.aL, aR = m.aR;
     const T Lslow = L.u - aL, Lfast = L.u + aL;
     const T Rslow = R.u - aR, Rfast = R.u + aR;
     T l1 = us - as, l4 = us + as;
@@ -570,8 +810,8 @@ __host__ __device__ inline Q4T<T> hlll_flux(const PrimT<T>& L, const PrimT<T>& R
     // ConservativeState(state=W): PrimitiveConverter.to_conservative (concrete_defs.py:126-141)
     const T ekL = (0.5 * L.r) * (L.u * L.u + L.v * L.v);
     const T ekR = (0.5 * R.r) * (R.u * R.u + R.v * R.v);
-    const T UL0 = L.r, UL1 = L.r * L.u, UL2 = L.r * L.v, UL3 = L.p / ph.gm1 + ekL;
-    const T UR0 = R.r, UR1 = R.r * R.u, UR2 = R.r * R.v, UR3 = R.p / ph.gm1 + ekR;
+    const T UL0 = L.r, UL1 = L.r * L.u, UL2 = L.r * L.v, UL3 = m.eL + ekL;
+    const T UR0 = R.r, UR1 = R.r * R.u, UR2 = R.r * R.v, UR3 = m.eR + ekR;
     // PrimitiveState.F(U=...) (states/primitive.py:203-209)
     const T FL0 = UL1, FL1 = UL1 * L.u + L.p, FL2 = UL1 * L.v, FL3 = L.u * (UL3 + L.p);
     const T FR0 = UR1, FR1 = UR1 * R.u + R.p, FR2 = UR1 * R.v, FR3 = R.u * (UR3 + R.p);
@@ -592,18 +832,20 @@ __host__ __device__ inline Q4T<T> hlll_flux(const PrimT<T>& L, const PrimT<T>& R
         const T mx = (ra >= rb) ? ra : rb;            // np.maximum(u/Lm, u/Lp)
         const T coef = Lminus * Lplus * (1.0 - alpha * (1.0 - mx));
         const T w = Lplus - Lminus;
-        F.v[0] = (Lplus * FL0 - Lminus * FR0 + coef * dU0) / w;
-        F.v[1] = (Lplus * FL1 - Lminus * FR1 + coef * dU1) / w;
-        F.v[2] = (Lplus * FL2 - Lminus * FR2 + coef * dU2) / w;
-        F.v[3] = (Lplus * FL3 - Lminus * FR3 + coef * dU3) / w;
+        T N[4];
+        N[0] = Lplus * FL0 - Lminus * FR0 + coef * dU0;
+        N[1] = Lplus * FL1 - Lminus * FR1 + coef * dU1;
+        N[2] = Lplus * FL2 - Lminus * FR2 + coef * dU2;
+        N[3] = Lplus * FL3 - Lminus * FR3 + coef * dU3;
+        div_all(N, w, F.v);
     }
     return F;
 }
 
 template <int FLUX, class T>
 __host__ __device__ inline Q4T<T> face_flux(const Q4T<T>& qL, const Q4T<T>& qR, const Phys& ph) {
-    const PrimT<T> L = cons_to_prim(qL, ph);
-    const PrimT<T> R = cons_to_prim(qR, ph);
+    PrimT<T> L, R;
+    cons_to_prim2(qL, qR, ph, L, R);
     if (FLUX == 0) return roe_flux(L, R, ph);
     return hlll_flux(L, R, ph);
 }
@@ -632,6 +874,7 @@ struct CellGeo {
     double xlE, xlW, xlN, xlS, ylE, ylW, ylN, ylS;
     double ainv;
     double dxE, dxW, dxN, dxS, dyE, dyW, dyN, dyS;
+    bool odd = false;  // a weight or offset beyond 2^60 (or not finite): limit_venkat takes the general path
 };
 
 template <class T>
@@ -716,6 +959,133 @@ __host__ __device__ inline double venkat_face(double dmax, double dmin, double d
     return limit_face<false>(dmax, dmin, d, 0);
 }
 
+// Stencil extrema: v_max_f64 / v_min_f64 as they are.  fmax and fmin of loaded values each first pass
+// every operand through a v_max_f64 x, x of its own, which only quiets signaling NaNs; a neighbour
+// that holds a NaN of either kind makes the gradient and with it the limited states NaN.
+__host__ __device__ inline double vmax(double a, double b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+#else
+    return fmax(a, b);
+#endif
+}
+__host__ __device__ inline double vmin(double a, double b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+#else
+    return fmin(a, b);
+#endif
+}
+__host__ __device__ inline double vmin_abs4(double a, double b, double c, double d) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    double r, t;
+    asm("v_min_f64 %0, |%1|, |%2|" : "=v"(r) : "v"(a), "v"(b));
+    asm("v_min_f64 %0, |%1|, |%2|" : "=v"(t) : "v"(c), "v"(d));
+    return vmin(r, t);
+#else
+    return fmin(fmin(fabs(a), fabs(b)), fmin(fabs(c), fabs(d)));
+#endif
+}
+template <class T>
+__host__ __device__ inline T vmax(T a, T b) { return fmax(a, b); }
+template <class T>
+__host__ __device__ inline T vmin(T a, T b) { return fmin(a, b); }
+
+// Venkatakrishnan's value for a slope s >= 0 of at most 2^495: both divisions' operands in range
+__host__ __device__ inline double venkat_in_range(double s) {
+    const double s2 = s * s;
+    return Recip(s2 + s + 2.0).div(s2 + 2.0 * s);
+}
+
+// n / d for a d that is 0 or in range: NaN for d = 0 (v_rcp_f64 gives an infinity, 1 - 0*inf NaN), which
+// fmin passes over
+__host__ __device__ inline double slope_or_nan(double n, double d) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return Recip(d).div(n);
+#else
+    return d == 0.0 ? __builtin_nan("") : n / d;
+#endif
+}
+
+// Limiter value of one variable of a cell: max(0, minimum over the four faces of Venkatakrishnan's value
+// of the face's slope) (Venkatakrishnan._venkata, limiters/limiters.py:38-49, np.minimum.reduce), from the
+// high-order terms h of the faces E, W, N, S (d = (u + h) - u).  3 divisions instead of 8, the same bits.
+//
+// The slopes of the faces with d > 0 are dmax/d, and division rounds monotonically, so the smallest
+// of them is dmax / max(d); likewise dmin / min(d) over d < 0.  phi(s) = (s^2 + 2s)/(s^2 + s + 2) rises
+// on [0, 4.8] (relative slope s phi'/phi >= 1/4 on [0, 2]), passes phi(2) = 1 and stays >= 1 beyond.  Its
+// computed value is within 6 units of 2^-53, so of two slopes that differ by more than 2^-40 of
+// themselves the smaller one has the smaller computed value as long as it is at most 2 (at
+// s = 2 exactly phi = 1 exactly, and no computed value of a larger slope is below 1).  So the value at
+// the smallest slope is the minimum unless another slope lies within 2^-40 of it, or all four exceed
+// 2: a wave with such a lane compares all four values.  A face with d = 0 has the slope 1, whose value
+// 3/4 enters as a constant.
+//
+// In-range divisions: dmax - dmin <= 2^100 and 2^-340 <= |u| < 2^101 make every non-zero difference
+// of the stencil and every non-zero d at least 2^-394 (each is a multiple of half the last place of
+// |u|), geometry up to 2^60 makes |d| <= 2^286, so a slope is 0 or in [2^-680, 2^496] and its
+// square does not overflow.  Where u is 0 the differences are tested themselves: a slope that
+// overflows gives inf/inf = NaN in the general evaluation, so a tiny d must not be passed over.  A
+// wave with a lane outside these ranges takes the general evaluation of all faces.
+__host__ __device__ __forceinline__ double limit_venkat(double u, double dmax, double dmin, const double (&h)[4], bool odd) {
+    const double dE = (u + h[0]) - u, dW = (u + h[1]) - u, dN = (u + h[2]) - u, dS = (u + h[3]) - u;
+    const double a = vmax(dE, dW), b = vmin(dE, dW), c = vmax(dN, dS), e = vmin(dN, dS);
+    const double P = vmax(a, c), p = vmin(a, c), M = vmin(b, e), m = vmax(b, e);  // the four d again
+    if (PHX_RARE(wave_lanes(vmax(P, -M) > 0.0) == 0)) return 0.75;  // flat: no increment at any face
+    const double near = 1.0 - 0x1p-40;
+    const double Pc = vmax(P, 0.0), Mc = vmin(M, 0.0);
+    const double sP = slope_or_nan(dmax, Pc), sM = slope_or_nan(dmin, Mc);
+    const double s = vmin(sP, sM);
+    const double cap = vmin_abs4(P, p, M, m) == 0.0 ? 0.75 : __builtin_inf();
+    const unsigned long long close = wave_lanes(vmax(p, m) > Pc * near) | wave_lanes(vmin(p, m) < Mc * near) |
+                                     wave_lanes(fabs(sP - sM) <= s * 0x1p-40) | wave_lanes(vmin(s, cap) > 2.0);
+    const double phi = vmin(venkat_in_range(s), cap);
+    // high words: |u| in [2^-340, 2^100 (1 + 2^-20)], the spread of the stencil at most that (a NaN is beyond)
+    const unsigned size = (hi_word(u) & 0x7fffffffu) - 0x2ab00000u, spread = hi_word(dmax - dmin);
+    const unsigned long long wide = wave_lanes(spread > 0x46300000u), off = wave_lanes(size > 0x46300000u - 0x2ab00000u);
+    if (PHX_USUAL(!odd & ((close | wide | off) == 0))) return phi;
+
+    double w = u;
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+v"(w));  // the increments again, not kept in registers from above
+#endif
+    double d[4];
+    int zero = (int)(u == 0.0) & zero_or_from(dmax, 0x1p-394) & zero_or_from(dmin, 0x1p-394);
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+        d[f] = (w + h[f]) - w;
+        zero &= zero_or_from(d[f], 0x1p-394);
+    }
+    if (!odd & ((wide | (off & wave_lanes(zero == 0))) == 0)) {
+        if (close == 0) return phi;
+        double x = cap;
+#pragma unroll
+        for (int f = 0; f < 4; ++f) x = vmin(x, venkat_in_range(slope_or_nan(d[f] > 0.0 ? dmax : dmin, d[f])));
+        return x;
+    }
+    const double pE = limit_face<false>(dmax, dmin, d[0], 0), pW = limit_face<false>(dmax, dmin, d[1], 0);
+    const double pN = limit_face<false>(dmax, dmin, d[2], 0), pS = limit_face<false>(dmax, dmin, d[3], 0);
+    const double x = limiter_min4<false>(pE, pW, pN, pS);
+    return (x < 0.0) ? 0.0 : x;
+}
+// The general form: any scalar type, with GEN the limiter `lim`.
+template <bool GEN, class T>
+__host__ __device__ inline T limit_cell(const T& u, const T& dmax, const T& dmin, const T (&h)[4], bool odd, int lim) {
+    if constexpr (std::is_same<T, double>::value) {
+        if (!GEN || lim == 0) return limit_venkat(u, dmax, dmin, h, odd);
+    }
+    const T pE = limit_face<GEN>(dmax, dmin, (u + h[0]) - u, lim);
+    const T pW = limit_face<GEN>(dmax, dmin, (u + h[1]) - u, lim);
+    const T pN = limit_face<GEN>(dmax, dmin, (u + h[2]) - u, lim);
+    const T pS = limit_face<GEN>(dmax, dmin, (u + h[3]) - u, lim);
+    const T phi = limiter_min4<GEN>(pE, pW, pN, pS);
+    return (phi < 0.0) ? T(0.0) : phi;                 // np.where(phi < 0, 0, phi)
+}
+
 // One cell of the second-order reconstruction (reconstruct_var: one conserved variable):
 //  * interface averages (blocks/quad_block.py:181-218),
 //  * Green-Gauss gradient (gradients/greengauss.py:134-155),
@@ -733,25 +1103,15 @@ __host__ __device__ inline void reconstruct_var(T u, T uw, T ue, T us, T un, con
     const T s = 0.5 * (us + u);
     const T gx = (e * g.xlE + w * g.xlW + n * g.xlN + s * g.xlS) * g.ainv;
     const T gy = (e * g.ylE + w * g.ylW + n * g.ylN + s * g.ylS) * g.ainv;
-    const T hE = gx * g.dxE + gy * g.dyE;
-    const T hW = gx * g.dxW + gy * g.dyW;
-    const T hN = gx * g.dxN + gy * g.dyN;
-    const T hS = gx * g.dxS + gy * g.dyS;
+    const T h[4] = {gx * g.dxE + gy * g.dyE, gx * g.dxW + gy * g.dyW, gx * g.dxN + gy * g.dyN, gx * g.dxS + gy * g.dyS};
     // np.maximum.reduce((U, UW, UE, US, UN)) - U
-    const T mx = fmax(fmax(fmax(fmax(u, uw), ue), us), un);
-    const T mn = fmin(fmin(fmin(fmin(u, uw), ue), us), un);
-    const T dmax = mx - u;
-    const T dmin = mn - u;
-    const T pE = limit_face<GEN>(dmax, dmin, (u + hE) - u, lim);
-    const T pW = limit_face<GEN>(dmax, dmin, (u + hW) - u, lim);
-    const T pN = limit_face<GEN>(dmax, dmin, (u + hN) - u, lim);
-    const T pS = limit_face<GEN>(dmax, dmin, (u + hS) - u, lim);
-    T phi = limiter_min4<GEN>(pE, pW, pN, pS);
-    phi = (phi < 0.0) ? T(0.0) : phi;                  // np.where(phi < 0, 0, phi)
-    qE = u + phi * hE;
-    qW = u + phi * hW;
-    qN = u + phi * hN;
-    qS = u + phi * hS;
+    const T mx = vmax(vmax(vmax(vmax(u, uw), ue), us), un);
+    const T mn = vmin(vmin(vmin(vmin(u, uw), ue), us), un);
+    const T phi = limit_cell<GEN>(u, T(mx - u), T(mn - u), h, g.odd, lim);
+    qE = u + phi * h[0];
+    qW = u + phi * h[1];
+    qN = u + phi * h[2];
+    qS = u + phi * h[3];
 }
 
 template <bool GEN = false, class T>

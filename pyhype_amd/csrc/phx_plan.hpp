@@ -11,6 +11,9 @@
 #include "phx_device.hpp"
 
 namespace phx {
+namespace stage {
+struct DevItem;  // a work item with its block's descriptor (phx_stage.hpp)
+}
 namespace host {
 
 constexpr int MAX_OUT = 8;  // outputs of one stage program (stage state + accumulators)
@@ -73,7 +76,7 @@ struct phx_plan {
     int64_t state_len = 0;
     int rows_per_item = 32, grid_waves = 0, waves_per_simd = 2;
     std::vector<phx::host::WorkItem> items[2];  // [0] general, [1] cartesian
-    phx::host::WorkItem* ditems[2] = {nullptr, nullptr};
+    phx::stage::DevItem* ditems[2] = {nullptr, nullptr};
     int grid[2] = {0, 0};
     // stage variant: 0 = fused rolling rows, 1 = split (reconstruct + x-faces, y-faces, update),
     // 2 = shared-halo workgroups, 3 = element-wise (cell-variable lanes, face lanes, cell lanes),
@@ -83,21 +86,21 @@ struct phx_plan {
     int variant = 0, rows_b = 8;
     std::vector<phx::host::WorkItem> items_b[2];  // split variant: update kernel
     int flat_q[2] = {0, 0};                          // variant 8: LDS faces per lane of the update kernel
-    phx::host::WorkItem* ditems_b[2] = {nullptr, nullptr};
+    phx::stage::DevItem* ditems_b[2] = {nullptr, nullptr};
     int grid_b[2] = {0, 0};
     std::vector<phx::host::WorkItem> items_f[2];  // variant 1: y-face kernel; variant 7: reconstruction
-    phx::host::WorkItem* ditems_f[2] = {nullptr, nullptr};
+    phx::stage::DevItem* ditems_f[2] = {nullptr, nullptr};
     int grid_f[2] = {0, 0};
     // element-wise variant: tiles of [0] the reconstruction (cells), [1] the faces, [2] the update (cells)
     std::vector<phx::host::WorkItem> items_e[3][2];
-    phx::host::WorkItem* ditems_e[3][2] = {};
+    phx::stage::DevItem* ditems_e[3][2] = {};
     // element-wise stage on a mesh with both geometry kinds: each phase's items of both kinds in one
     // list (one launch; the kernels pick the geometry path per block)
-    phx::host::WorkItem* ditems_em[3] = {};
+    phx::stage::DevItem* ditems_em[3] = {};
     int n_em[3] = {0, 0, 0}, grid_em[3] = {0, 0, 0};
     // split stages 6 and 7 likewise: merged lists of items (variant 6 reconstruction), items_b (y-faces
     // and update) and items_f (variant 7 reconstruction)
-    phx::host::WorkItem* ditems_m[3] = {};
+    phx::stage::DevItem* ditems_m[3] = {};
     int n_m[3] = {0, 0, 0}, grid_m[3] = {0, 0, 0};
     int grid_e[3][2] = {};
     double* ew_rb = nullptr;  // element-wise variant: limited face states E, W, N, S per cell (16 doubles)

@@ -44,13 +44,21 @@ __device__ __forceinline__ int wave_slot(int nslot) {
     return (int)((blockIdx.x * (blockDim.x / WAVE) + threadIdx.x / WAVE) & (nslot - 1));
 }
 
+// A work item as the kernels read it: with the descriptor of its block, so that the first values a
+// wave computes addresses from arrive after one scalar load instead of two in a row (about 0.2 us of
+// every launch, more where the descriptors are not in the cache yet).
+struct DevItem {
+    int block, j0, r0, r1;
+    DevBlock b;
+};
+
 // Every per-item function below is __forceinline__, so that no kernel makes a device-function call.
 // Outlined (s_swappc) item functions of the HLLL Gauss-face and generic shared-halo kernels, which
 // appeared when the HLLL norm grew, returned NaN residuals on gfx950 (ROCm 7.2) where the same
 // source inlined, and a stand-alone kernel of the same flux, are bit-exact.
 struct StageArgs {
     const DevBlock* blocks;
-    const WorkItem* items;
+    const DevItem* items;
     int nitems;
     int nout;
     int state_out;
@@ -81,6 +89,14 @@ struct StageArgs {
 template <class T>
 __device__ __forceinline__ const T& const_ref(const T* p, long i) {
     return *(const T*)(((const __attribute__((address_space(4))) T*)p) + i);
+}
+
+// Whether the block's case became unrealizable at an earlier step: it is frozen, as the reference aborts
+// that run (Euler2D.py:144-152).  Scalar loads (a lane that fails in this stage writes the current step,
+// which leaves the comparison as it is); a kernel asks after it has issued its first loads, which do
+// not wait for the answer then.
+__device__ __forceinline__ bool frozen_case(const StageArgs& A, const DevBlock& B) {
+    return A.skip_dead && ld_const(A.bad, B.case_id) < ld_const(A.step, 0);
 }
 
 // cross-lane moves of a 4-vector
@@ -192,10 +208,10 @@ __device__ __forceinline__ void reduce_item(const StageArgs& A, const DevBlock& 
 // blocks the column arrays are loaded once per item and the cell areas one row ahead, so the only
 // geometry a row iteration waits for was requested an iteration earlier.
 template <bool CART, int FLUX, bool GEN, bool PF = false>
-__device__ __forceinline__ void stage_item(const StageArgs& A, const WorkItem it) {
-    const DevBlock& B = PF ? const_ref(A.blocks, it.block) : A.blocks[it.block];
+__device__ __forceinline__ void stage_item(const StageArgs& A, const DevItem& it) {
+    const DevBlock& B = PF ? it.b : A.blocks[it.block];
     // a case that became unrealizable is frozen: the reference aborts that run (Euler2D.py:144-152)
-    if (A.skip_dead && A.bad[B.case_id] < *A.step) return;
+    if (frozen_case(A, B)) return;
     const int lane = threadIdx.x & (WAVE - 1);
     const int nx = B.nx, ny = B.ny;
     const int j = it.j0 - HALO + lane;
@@ -281,7 +297,8 @@ __device__ __forceinline__ void stage_item(const StageArgs& A, const WorkItem it
                 const int kk = k - 1;
                 Q4 Res;
 #pragma unroll
-                for (int c = 0; c < 4; ++c) Res.v[c] = (0.5 * (part.v[c] - prevLN * (2.0 * F.v[c]))) / prevA;
+                for (int c = 0; c < 4; ++c) Res.v[c] = 0.5 * (part.v[c] - prevLN * (2.0 * F.v[c]));
+                phx::div_all(Res.v, prevA, Res.v);
                 emit_row<CART, PF>(A, B, kk, j, dt, Res, lane_dt, lane_bad, pre, cols.dx);
             }
             if (xrow) {
@@ -324,7 +341,7 @@ template <bool CART, int FLUX, int MINW, bool GEN>
 __global__ void __launch_bounds__(WAVE, MINW) k_stage(StageArgs A) {
     int lo, hi, first, stride;
     item_range(A.nitems, lo, hi, first, stride);
-    for (int i = first; i < hi; i += stride) stage_item<CART, FLUX, GEN, MINW == 2>(A, ld_const(A.items, i));
+    for (int i = first; i < hi; i += stride) stage_item<CART, FLUX, GEN, MINW == 2>(A, const_ref(A.items, i));
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -338,9 +355,9 @@ __global__ void __launch_bounds__(WAVE, MINW) k_stage(StageArgs A) {
 constexpr int WGW = 4;
 
 template <bool CART, int FLUX, bool GEN>
-__device__ __forceinline__ void stage_wg_item(const StageArgs& A, const WorkItem it, Q4* lds_N, Q4* lds_F) {
+__device__ __forceinline__ void stage_wg_item(const StageArgs& A, const DevItem& it, Q4* lds_N, Q4* lds_F) {
     const DevBlock& B = A.blocks[it.block];
-    if (A.skip_dead && A.bad[B.case_id] < *A.step) return;  // uniform over the workgroup
+    if (frozen_case(A, B)) return;  // uniform over the workgroup
     const int lane = threadIdx.x & (WAVE - 1);
     const int w = threadIdx.x / WAVE;
     const int nx = B.nx, ny = B.ny;
@@ -411,7 +428,8 @@ __device__ __forceinline__ void stage_wg_item(const StageArgs& A, const WorkItem
                         } else {
                             Q4 Res;
 #pragma unroll
-                            for (int c = 0; c < 4; ++c) Res.v[c] = (0.5 * (part.v[c] - prevLN * (2.0 * F.v[c]))) / prevA;
+                            for (int c = 0; c < 4; ++c) Res.v[c] = 0.5 * (part.v[c] - prevLN * (2.0 * F.v[c]));
+                            phx::div_all(Res.v, prevA, Res.v);
                             emit_row<CART>(A, B, k - 1, j, dt, Res, lane_dt, lane_bad);
                         }
                     }
@@ -456,15 +474,16 @@ __device__ __forceinline__ void stage_wg_item(const StageArgs& A, const WorkItem
             Q4 Res;
 #pragma unroll
             for (int c = 0; c < 4; ++c)
-                Res.v[c] = (0.5 * ((first_part.v[c] + first_LS * (2.0 * FS_first.v[c])) - first_LN * (2.0 * FN.v[c]))) /
-                           first_A;
+                Res.v[c] = 0.5 * ((first_part.v[c] + first_LS * (2.0 * FS_first.v[c])) - first_LN * (2.0 * FN.v[c]));
+            phx::div_all(Res.v, first_A, Res.v);
             emit_row<CART>(A, B, a, j, dt, Res, lane_dt, lane_bad);
         }
         if (!top && !(single && !bottom)) {
             const Q4 FN = lds_F[(w + 1) * WAVE + lane];
             Q4 Res;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) Res.v[c] = (0.5 * (part.v[c] - prevLN * (2.0 * FN.v[c]))) / prevA;
+            for (int c = 0; c < 4; ++c) Res.v[c] = 0.5 * (part.v[c] - prevLN * (2.0 * FN.v[c]));
+            phx::div_all(Res.v, prevA, Res.v);
             emit_row<CART>(A, B, b - 1, j, dt, Res, lane_dt, lane_bad);
         }
     }
@@ -478,7 +497,7 @@ __global__ void __launch_bounds__(WGW * WAVE, MINW) k_stage_wg(StageArgs A) {
     int lo, hi, first, stride;
     item_range(A.nitems, lo, hi, first, stride);
     for (int i = first; i < hi; i += stride) {
-        stage_wg_item<CART, FLUX, GEN>(A, ld_const(A.items, i), lds_N, lds_F);
+        stage_wg_item<CART, FLUX, GEN>(A, const_ref(A.items, i), lds_N, lds_F);
         __syncthreads();  // the next item reuses the exchange buffers
     }
 }
@@ -537,8 +556,8 @@ __device__ __forceinline__ void emit_half(const StageArgs& A, const DevBlock& B,
 }
 
 template <bool CART, int FLUX, bool GEN, int H>
-__device__ __forceinline__ void stage_pair_body(const StageArgs& A, const WorkItem it, PairLds& L) {
-    const DevBlock& B = const_ref(A.blocks, it.block);
+__device__ __forceinline__ void stage_pair_body(const StageArgs& A, const DevItem& it, PairLds& L) {
+    const DevBlock& B = it.b;
     const int lane = threadIdx.x & (WAVE - 1);
     const int nx = B.nx, ny = B.ny;
     const int j = it.j0 - HALO + lane;
@@ -648,7 +667,8 @@ __device__ __forceinline__ void stage_pair_body(const StageArgs& A, const WorkIt
                 // residual of row k-1: 0.5*(W - E + S - N)/A with I = L*(2*F) (fvm/base.py:141-190)
                 double res[2];
 #pragma unroll
-                for (int i = 0; i < 2; ++i) res[i] = (0.5 * (part[i] - prevLN * (2.0 * fy[i]))) / prevA;
+                for (int i = 0; i < 2; ++i) res[i] = 0.5 * (part[i] - prevLN * (2.0 * fy[i]));
+                phx::div_all(res, prevA, res);
                 emit_half<CART, H>(A, B, k - 1, j, dt, res, o);
             }
             if (xrow) {
@@ -686,9 +706,9 @@ __global__ void __launch_bounds__(PAIR_WAVES * WAVE, MINW) k_stage_pair(StageArg
     int lo, hi, first, stride;
     item_range(A.nitems, lo, hi, first, stride);
     for (int i = first; i < hi; i += stride) {
-        const WorkItem it = ld_const(A.items, i);
-        const DevBlock& B = const_ref(A.blocks, it.block);
-        if (A.skip_dead && A.bad[B.case_id] < *A.step) continue;  // uniform over the workgroup
+        const DevItem& it = const_ref(A.items, i);
+        const DevBlock& B = it.b;
+        if (frozen_case(A, B)) continue;  // uniform over the workgroup
         if (h == 0) stage_pair_body<CART, FLUX, GEN, 0>(A, it, L);
         else stage_pair_body<CART, FLUX, GEN, 1>(A, it, L);
         __syncthreads();  // the next item reuses the exchange buffers
@@ -718,9 +738,9 @@ __device__ __forceinline__ void acc_w(Q4& acc, double w, const Q4& F) {
 }
 
 template <bool CART, int FLUX>
-__device__ __forceinline__ void recon_x_item_q(const StageArgs& A, const WorkItem it) {
+__device__ __forceinline__ void recon_x_item_q(const StageArgs& A, const DevItem& it) {
     const DevBlock& B = A.blocks[it.block];
-    if (A.skip_dead && A.bad[B.case_id] < *A.step) return;
+    if (frozen_case(A, B)) return;
     const int nx = B.nx;
     const int j = it.j0 - HALO + threadIdx.x % WAVE;
     const bool valid = (j >= -1) && (j <= nx);
@@ -811,9 +831,9 @@ __device__ __forceinline__ Q4 yface_sum_q(const StageArgs& A, const DevBlock& B,
 }
 
 template <bool CART, int FLUX>
-__device__ __forceinline__ void yface_item_q(const StageArgs& A, const WorkItem it) {
+__device__ __forceinline__ void yface_item_q(const StageArgs& A, const DevItem& it) {
     const DevBlock& B = A.blocks[it.block];
-    if (A.skip_dead && A.bad[B.case_id] < *A.step) return;
+    if (frozen_case(A, B)) return;
     const int nx = B.nx;
     const int j = it.j0 + (int)(threadIdx.x % WAVE);
     if (j >= nx) return;
@@ -824,9 +844,9 @@ __device__ __forceinline__ void yface_item_q(const StageArgs& A, const WorkItem 
 
 // Gauss faces, y-faces and update in one pass (variant 5; yface_update_item with the sums S_F)
 template <bool CART, int FLUX>
-__device__ __forceinline__ void yface_update_item_q(const StageArgs& A, const WorkItem it) {
+__device__ __forceinline__ void yface_update_item_q(const StageArgs& A, const DevItem& it) {
     const DevBlock& B = A.blocks[it.block];
-    if (A.skip_dead && A.bad[B.case_id] < *A.step) return;
+    if (frozen_case(A, B)) return;
     const int lane = threadIdx.x & (WAVE - 1);
     const int nx = B.nx;
     const int j = it.j0 + lane;
@@ -844,7 +864,8 @@ __device__ __forceinline__ void yface_update_item_q(const StageArgs& A, const Wo
             cell_L<CART>(B, k, j, LW, LE, LS, LN, Ac);
             Q4 Res;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) Res.v[c] = (0.5 * ((p.v[c] + LS * FS.v[c]) - LN * FN.v[c])) / Ac;
+            for (int c = 0; c < 4; ++c) Res.v[c] = 0.5 * ((p.v[c] + LS * FS.v[c]) - LN * FN.v[c]);
+            phx::div_all(Res.v, Ac, Res.v);
             emit_row<CART>(A, B, k, j, dt, Res, lane_dt, lane_bad);
             FS = FN;
         }
@@ -853,9 +874,8 @@ __device__ __forceinline__ void yface_update_item_q(const StageArgs& A, const Wo
 }
 
 template <bool CART, int FLUX, bool GEN>
-__device__ __forceinline__ void recon_x_item(const StageArgs& A, const WorkItem it) {
-    const DevBlock& B = const_ref(A.blocks, it.block);
-    if (A.skip_dead && A.bad[B.case_id] < *A.step) return;
+__device__ __forceinline__ void recon_x_item(const StageArgs& A, const DevItem& it) {
+    const DevBlock& B = it.b;
     const int nx = B.nx;
     const int j = it.j0 - HALO + threadIdx.x % WAVE;
     const bool valid = (j >= -1) && (j <= nx);
@@ -872,12 +892,16 @@ __device__ __forceinline__ void recon_x_item(const StageArgs& A, const WorkItem 
     for (int k = it.r0; k < it.r1; ++k) {
         if (inner) Up = fetch_r<CART, GEN>(A.blocks, B, A.Uin, k + 1, j, ph);
         else if (gcol && k + 1 < it.r1) Up = fetch_r<CART, GEN>(A.blocks, B, A.Uin, k + 1, j, ph);
+        phx::CellGeo g;
+        double LW, LE, LS, LN, Ac;
+        if (recon) g = cell_geo<CART>(B, k, j);
+        if (owner) cell_L<CART>(B, k, j, LW, LE, LS, LN, Ac);
+        if (frozen_case(A, B)) return;
         const Q4 Uw = shfl_up1(Uc);
         const Q4 Ue = shfl_down1(Uc);
         phx::Recon r;
         r.E = r.W = r.N = r.S = phx::q4zero();
         if (recon) {
-            const phx::CellGeo g = cell_geo<CART>(B, k, j);
             r = phx::reconstruct<GEN>(Uc, Uw, Ue, Um, Up, g, ph.limiter);
         }
         const Q4 qsend = (j == -1) ? Uc : r.E;
@@ -890,8 +914,6 @@ __device__ __forceinline__ void recon_x_item(const StageArgs& A, const WorkItem 
         }
         const Q4 FE = shfl_down1(FW);
         if (owner) {
-            double LW, LE, LS, LN, Ac;
-            cell_L<CART>(B, k, j, LW, LE, LS, LN, Ac);
             Q4 part;
 #pragma unroll
             for (int c = 0; c < 4; ++c) part.v[c] = LW * (2.0 * FW.v[c]) - LE * (2.0 * FE.v[c]);
@@ -908,9 +930,9 @@ __device__ __forceinline__ void recon_x_item(const StageArgs& A, const WorkItem 
 // y-faces of face rows [r0, r1) of a strip of 64 columns (face f between rows f-1 and f; f = 0 and
 // f = ny take the outer states of the S and N boundaries): one flux per lane and face, stored.
 template <bool CART, int FLUX, bool GEN>
-__device__ __forceinline__ void yface_item(const StageArgs& A, const WorkItem it) {
+__device__ __forceinline__ void yface_item(const StageArgs& A, const DevItem& it) {
     const DevBlock& B = A.blocks[it.block];
-    if (A.skip_dead && A.bad[B.case_id] < *A.step) return;
+    if (frozen_case(A, B)) return;
     const int nx = B.nx, ny = B.ny;
     const int j = it.j0 + (int)(threadIdx.x % WAVE);
     if (j >= nx) return;
@@ -929,9 +951,9 @@ __device__ __forceinline__ void yface_item(const StageArgs& A, const WorkItem it
 // residual ((x-part + LS*(2 F_S)) - LN*(2 F_N))/A (Gauss sums S_F in place of 2 F with nq > 1) of rows [r0, r1) of a 64-column strip, then every
 // Butcher output, the CFL quantity and realizability (as the fused kernel).
 template <bool CART>
-__device__ __forceinline__ void update_item(const StageArgs& A, const WorkItem it) {
+__device__ __forceinline__ void update_item(const StageArgs& A, const DevItem& it) {
     const DevBlock& B = A.blocks[it.block];
-    if (A.skip_dead && A.bad[B.case_id] < *A.step) return;
+    if (frozen_case(A, B)) return;
     const int lane = threadIdx.x & (WAVE - 1);
     const int nx = B.nx;
     const int j = it.j0 + lane;
@@ -949,11 +971,12 @@ __device__ __forceinline__ void update_item(const StageArgs& A, const WorkItem i
             Q4 Res;
             if (A.ph.nq > 1) {  // y-face entries are the Gauss sums already
 #pragma unroll
-                for (int c = 0; c < 4; ++c) Res.v[c] = (0.5 * ((p.v[c] + LS * FS.v[c]) - LN * FN.v[c])) / Ac;
+                for (int c = 0; c < 4; ++c) Res.v[c] = 0.5 * ((p.v[c] + LS * FS.v[c]) - LN * FN.v[c]);
+                phx::div_all(Res.v, Ac, Res.v);
             } else {
 #pragma unroll
-                for (int c = 0; c < 4; ++c)
-                    Res.v[c] = (0.5 * ((p.v[c] + LS * (2.0 * FS.v[c])) - LN * (2.0 * FN.v[c]))) / Ac;
+                for (int c = 0; c < 4; ++c) Res.v[c] = 0.5 * ((p.v[c] + LS * (2.0 * FS.v[c])) - LN * (2.0 * FN.v[c]));
+                phx::div_all(Res.v, Ac, Res.v);
             }
             emit_row<CART>(A, B, k, j, dt, Res, lane_dt, lane_bad);
             FS = FN;
@@ -979,9 +1002,9 @@ __device__ __forceinline__ Q4 yface_flux_at(const StageArgs& A, const DevBlock& 
 }
 
 template <bool CART, int FLUX, bool GEN>
-__device__ __forceinline__ void yface_update_item(const StageArgs& A, const WorkItem it) {
+__device__ __forceinline__ void yface_update_item(const StageArgs& A, const DevItem& it) {
     const DevBlock& B = A.blocks[it.block];
-    if (A.skip_dead && A.bad[B.case_id] < *A.step) return;
+    if (frozen_case(A, B)) return;
     const int lane = threadIdx.x & (WAVE - 1);
     const int nx = B.nx;
     const int j = it.j0 + lane;
@@ -999,8 +1022,8 @@ __device__ __forceinline__ void yface_update_item(const StageArgs& A, const Work
             cell_L<CART>(B, k, j, LW, LE, LS, LN, Ac);
             Q4 Res;
 #pragma unroll
-            for (int c = 0; c < 4; ++c)
-                Res.v[c] = (0.5 * ((p.v[c] + LS * (2.0 * FS.v[c])) - LN * (2.0 * FN.v[c]))) / Ac;
+            for (int c = 0; c < 4; ++c) Res.v[c] = 0.5 * ((p.v[c] + LS * (2.0 * FS.v[c])) - LN * (2.0 * FN.v[c]));
+            phx::div_all(Res.v, Ac, Res.v);
             emit_row<CART>(A, B, k, j, dt, Res, lane_dt, lane_bad);
             FS = FN;
         }
@@ -1016,15 +1039,27 @@ constexpr int YU_MAX_ROWS = 7;  // rows per item (R + 1 <= 8 waves per workgroup
 
 // Q = true: Gauss faces (the sums S_F of yface_sum_q, the residual of the nq-point rule)
 template <bool CART, int FLUX, bool GEN, bool Q>
-__device__ __forceinline__ void yface_update_wg_item(const StageArgs& A, const WorkItem it, Q4* lds) {
-    const DevBlock B = ld_const(A.blocks, it.block);  // descriptor in scalar registers
-    if (A.skip_dead && A.bad[B.case_id] < *A.step) return;  // uniform over the workgroup
+__device__ __forceinline__ void yface_update_wg_item(const StageArgs& A, const DevItem& it, Q4* lds) {
+    const DevBlock B = it.b;  // in scalar registers
     const int lane = threadIdx.x & (WAVE - 1);
     const int w = threadIdx.x / WAVE;
     const int nx = B.nx;
     const int j = it.j0 + lane;
     const int nrow = it.r1 - it.r0;
     const Phys ph = A.ph;
+#ifdef YPRE
+    // the cell's own values with the face states: they arrive while the flux is computed
+    const bool own = w < nrow && j < nx;
+    Q4 p, pre[EMIT_CHUNK];
+    double LW, LE, LS, LN, Ac;
+    if (own) {
+        p = ld4(A.p1 + B.off + 4 * ((long)(it.r0 + w) * nx + j));
+        cell_L<CART>(B, it.r0 + w, j, LW, LE, LS, LN, Ac);
+        if (YPRE > 1) prefetch_sources(A, B, it.r0 + w, j, pre);
+    }
+#endif
+    const bool dead = frozen_case(A, B);
+    if (dead) return;  // uniform over the workgroup
     if (w <= nrow && j < nx) {
         if (Q) lds[w * WAVE + lane] = yface_sum_q<CART, FLUX>(A, B, A.sn + 2 * ph.nq * B.off, it.r0 + w, j, ph);
         else lds[w * WAVE + lane] = yface_flux_at<CART, FLUX, GEN>(A, B, A.sn + 2 * B.off, it.r0 + w, j, ph);
@@ -1036,17 +1071,20 @@ __device__ __forceinline__ void yface_update_wg_item(const StageArgs& A, const W
         const int k = it.r0 + w;
         const double dt = (A.dt != nullptr) ? ld_const(A.dt, B.case_id) : 0.0;
         const Q4 FS = lds[w * WAVE + lane], FN = lds[(w + 1) * WAVE + lane];
+#ifndef YPRE
         const Q4 p = ld4(A.p1 + B.off + 4 * ((long)k * nx + j));
         double LW, LE, LS, LN, Ac;
         cell_L<CART>(B, k, j, LW, LE, LS, LN, Ac);
+#endif
         Q4 Res;
         if (Q) {  // the face entries are the Gauss sums already
 #pragma unroll
-            for (int c = 0; c < 4; ++c) Res.v[c] = (0.5 * ((p.v[c] + LS * FS.v[c]) - LN * FN.v[c])) / Ac;
+            for (int c = 0; c < 4; ++c) Res.v[c] = 0.5 * ((p.v[c] + LS * FS.v[c]) - LN * FN.v[c]);
+            phx::div_all(Res.v, Ac, Res.v);
         } else {
 #pragma unroll
-            for (int c = 0; c < 4; ++c)
-                Res.v[c] = (0.5 * ((p.v[c] + LS * (2.0 * FS.v[c])) - LN * (2.0 * FN.v[c]))) / Ac;
+            for (int c = 0; c < 4; ++c) Res.v[c] = 0.5 * ((p.v[c] + LS * (2.0 * FS.v[c])) - LN * (2.0 * FN.v[c]));
+            phx::div_all(Res.v, Ac, Res.v);
         }
         emit_row<CART>(A, B, k, j, dt, Res, lane_dt, lane_bad);
     }
@@ -1061,9 +1099,9 @@ __global__ void __launch_bounds__((YU_MAX_ROWS + 1) * WAVE) k_yface_update_wg(St
     int lo, hi, first, stride;
     item_range(A.nitems, lo, hi, first, stride);
     for (int i = first; i < hi; i += stride) {
-        const WorkItem it = ld_const(A.items, i);
+        const DevItem& it = const_ref(A.items, i);
         if (CK == 2) {
-            if (ld_const(A.blocks, it.block).kind == PHX_GEOM_CARTESIAN) yface_update_wg_item<true, FLUX, GEN, Q>(A, it, lds);
+            if (it.b.kind == PHX_GEOM_CARTESIAN) yface_update_wg_item<true, FLUX, GEN, Q>(A, it, lds);
             else yface_update_wg_item<false, FLUX, GEN, Q>(A, it, lds);
         } else {
             yface_update_wg_item<CK == 1, FLUX, GEN, Q>(A, it, lds);
@@ -1081,9 +1119,9 @@ __global__ void __launch_bounds__((YU_MAX_ROWS + 1) * WAVE) k_yface_update_wg(St
 // range).  T = (A.rows_wave + 1) * WAVE; the host sizes the ranges so that n + nx <= A.fq * T, the
 // faces the dynamic LDS holds.
 template <bool CART, int FLUX, bool GEN>
-__device__ __forceinline__ void yface_update_flat_item(const StageArgs& A, const WorkItem it, Q4* lds) {
-    const DevBlock B = ld_const(A.blocks, it.block);  // descriptor in scalar registers
-    if (A.skip_dead && A.bad[B.case_id] < *A.step) return;  // uniform over the workgroup
+__device__ __forceinline__ void yface_update_flat_item(const StageArgs& A, const DevItem& it, Q4* lds) {
+    const DevBlock B = it.b;  // in scalar registers
+    if (frozen_case(A, B)) return;  // uniform over the workgroup
     const int T = blockDim.x;
     const int t = threadIdx.x;
     const int lane = t & (WAVE - 1);
@@ -1109,8 +1147,8 @@ __device__ __forceinline__ void yface_update_flat_item(const StageArgs& A, const
         cell_L<CART>(B, k, j, LW, LE, LS, LN, Ac);
         Q4 Res;
 #pragma unroll
-        for (int cc = 0; cc < 4; ++cc)
-            Res.v[cc] = (0.5 * ((p.v[cc] + LS * (2.0 * FS.v[cc])) - LN * (2.0 * FN.v[cc]))) / Ac;
+        for (int cc = 0; cc < 4; ++cc) Res.v[cc] = 0.5 * ((p.v[cc] + LS * (2.0 * FS.v[cc])) - LN * (2.0 * FN.v[cc]));
+        phx::div_all(Res.v, Ac, Res.v);
         emit_row<CART>(A, B, k, j, dt, Res, lane_dt, lane_bad);
     }
     reduce_item(A, B, lane, lane_dt, lane_bad);
@@ -1124,7 +1162,7 @@ __global__ void __launch_bounds__(FLAT_MAX_WAVES * WAVE) k_yface_update_flat(Sta
     int lo, hi, first, stride;
     item_range(A.nitems, lo, hi, first, stride);
     for (int i = first; i < hi; i += stride) {
-        yface_update_flat_item<CART, FLUX, GEN>(A, ld_const(A.items, i), flat_lds);
+        yface_update_flat_item<CART, FLUX, GEN>(A, const_ref(A.items, i), flat_lds);
         __syncthreads();  // the next item reuses the face buffer
     }
 }
@@ -1133,7 +1171,7 @@ template <bool CART, int FLUX, bool GEN>
 __global__ void __launch_bounds__(WAVE) k_yface_update(StageArgs A) {
     int lo, hi, first, stride;
     item_range(A.nitems, lo, hi, first, stride);
-    for (int i = first; i < hi; i += stride) yface_update_item<CART, FLUX, GEN>(A, ld_const(A.items, i));
+    for (int i = first; i < hi; i += stride) yface_update_item<CART, FLUX, GEN>(A, const_ref(A.items, i));
 }
 
 template <int CK, int FLUX, int MINW, bool GEN>
@@ -1141,9 +1179,9 @@ __global__ void __launch_bounds__(WAVE, MINW) k_recon_x(StageArgs A) {
     int lo, hi, first, stride;
     item_range(A.nitems, lo, hi, first, stride);
     for (int i = first; i < hi; i += stride) {
-        const WorkItem it = ld_const(A.items, i);
+        const DevItem& it = const_ref(A.items, i);
         if (CK == 2) {
-            if (ld_const(A.blocks, it.block).kind == PHX_GEOM_CARTESIAN) recon_x_item<true, FLUX, GEN>(A, it);
+            if (it.b.kind == PHX_GEOM_CARTESIAN) recon_x_item<true, FLUX, GEN>(A, it);
             else recon_x_item<false, FLUX, GEN>(A, it);
         } else {
             recon_x_item<CK == 1, FLUX, GEN>(A, it);
@@ -1163,9 +1201,8 @@ __global__ void __launch_bounds__(WAVE, MINW) k_recon_x(StageArgs A) {
 constexpr int LIN_OWN = WAVE - 2;
 
 template <bool CART, int FLUX, bool GEN>
-__device__ __forceinline__ void recon_x_lin_item(const StageArgs& A, const WorkItem it) {
-    const DevBlock B = ld_const(A.blocks, it.block);  // descriptor in scalar registers
-    if (A.skip_dead && A.bad[B.case_id] < *A.step) return;
+__device__ __forceinline__ void recon_x_lin_item(const StageArgs& A, const DevItem& it) {
+    const DevBlock B = it.b;  // in scalar registers
     const int nx = B.nx, npos = B.ny * (nx + 1);
     const int lane = threadIdx.x % WAVE;
     const int p = it.j0 - 1 + lane;
@@ -1186,6 +1223,13 @@ __device__ __forceinline__ void recon_x_lin_item(const StageArgs& A, const WorkI
     }
     if (wmem) Uw = fetch_r<CART, GEN>(A.blocks, B, A.Uin, k, j - 1, ph);
     if (emem) Ue = fetch_r<CART, GEN>(A.blocks, B, A.Uin, k, j + 1, ph);
+    phx::CellGeo g;
+    double LW, LE, LS, LN, Ac;
+    if (cell) {
+        g = cell_geo<CART>(B, k, j);
+        cell_L<CART>(B, k, j, LW, LE, LS, LN, Ac);
+    }
+    if (frozen_case(A, B)) return;
     const Q4 Uwl = shfl_up1(Uc);
     const Q4 Uel = shfl_down1(Uc);
     if (!wmem) Uw = Uwl;
@@ -1193,7 +1237,6 @@ __device__ __forceinline__ void recon_x_lin_item(const StageArgs& A, const WorkI
     phx::Recon r;
     r.E = r.W = r.N = r.S = phx::q4zero();
     if (cell) {
-        const phx::CellGeo g = cell_geo<CART>(B, k, j);
         r = phx::reconstruct<GEN>(Uc, Uw, Ue, Um, Up, g, ph.limiter);
     }
     const Q4 QEl = shfl_up1(r.E);  // limited east state of position p-1 (cell j-1 of the same row for j > 0)
@@ -1205,8 +1248,6 @@ __device__ __forceinline__ void recon_x_lin_item(const StageArgs& A, const WorkI
     }
     const Q4 FE = shfl_down1(FW);
     if (cell && lane > 0 && lane < WAVE - 1) {
-        double LW, LE, LS, LN, Ac;
-        cell_L<CART>(B, k, j, LW, LE, LS, LN, Ac);
         Q4 part;
 #pragma unroll
         for (int c = 0; c < 4; ++c) part.v[c] = LW * (2.0 * FW.v[c]) - LE * (2.0 * FE.v[c]);
@@ -1222,9 +1263,9 @@ __global__ void __launch_bounds__(WAVE, MINW) k_recon_x_lin(StageArgs A) {
     int lo, hi, first, stride;
     item_range(A.nitems, lo, hi, first, stride);
     for (int i = first; i < hi; i += stride) {
-        const WorkItem it = ld_const(A.items, i);
+        const DevItem& it = const_ref(A.items, i);
         if (CK == 2) {
-            if (ld_const(A.blocks, it.block).kind == PHX_GEOM_CARTESIAN) recon_x_lin_item<true, FLUX, GEN>(A, it);
+            if (it.b.kind == PHX_GEOM_CARTESIAN) recon_x_lin_item<true, FLUX, GEN>(A, it);
             else recon_x_lin_item<false, FLUX, GEN>(A, it);
         } else {
             recon_x_lin_item<CK == 1, FLUX, GEN>(A, it);
@@ -1236,7 +1277,7 @@ template <bool CART, int FLUX, bool GEN>
 __global__ void __launch_bounds__(WAVE) k_yface(StageArgs A) {
     int lo, hi, first, stride;
     item_range(A.nitems, lo, hi, first, stride);
-    for (int i = first; i < hi; i += stride) yface_item<CART, FLUX, GEN>(A, ld_const(A.items, i));
+    for (int i = first; i < hi; i += stride) yface_item<CART, FLUX, GEN>(A, const_ref(A.items, i));
 }
 
 // Gauss faces (nq > 1): kernels of their own, so that the register budget of the 1-point kernels is
@@ -1245,28 +1286,28 @@ template <bool CART, int FLUX>
 __global__ void __launch_bounds__(WAVE, 2) k_recon_x_q(StageArgs A) {
     int lo, hi, first, stride;
     item_range(A.nitems, lo, hi, first, stride);
-    for (int i = first; i < hi; i += stride) recon_x_item_q<CART, FLUX>(A, ld_const(A.items, i));
+    for (int i = first; i < hi; i += stride) recon_x_item_q<CART, FLUX>(A, const_ref(A.items, i));
 }
 
 template <bool CART, int FLUX>
 __global__ void __launch_bounds__(WAVE) k_yface_q(StageArgs A) {
     int lo, hi, first, stride;
     item_range(A.nitems, lo, hi, first, stride);
-    for (int i = first; i < hi; i += stride) yface_item_q<CART, FLUX>(A, ld_const(A.items, i));
+    for (int i = first; i < hi; i += stride) yface_item_q<CART, FLUX>(A, const_ref(A.items, i));
 }
 
 template <bool CART, int FLUX>
 __global__ void __launch_bounds__(WAVE) k_yface_update_q(StageArgs A) {
     int lo, hi, first, stride;
     item_range(A.nitems, lo, hi, first, stride);
-    for (int i = first; i < hi; i += stride) yface_update_item_q<CART, FLUX>(A, ld_const(A.items, i));
+    for (int i = first; i < hi; i += stride) yface_update_item_q<CART, FLUX>(A, const_ref(A.items, i));
 }
 
 template <bool CART>
 __global__ void __launch_bounds__(WAVE) k_update(StageArgs A) {
     int lo, hi, first, stride;
     item_range(A.nitems, lo, hi, first, stride);
-    for (int i = first; i < hi; i += stride) update_item<CART>(A, ld_const(A.items, i));
+    for (int i = first; i < hi; i += stride) update_item<CART>(A, const_ref(A.items, i));
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1294,9 +1335,9 @@ __device__ __forceinline__ double ew_value(const StageArgs& A, const DevBlock& B
 }
 
 template <bool CART, bool GEN>
-__device__ __forceinline__ void ew_recon_tile(const StageArgs& A, const WorkItem it) {
+__device__ __forceinline__ void ew_recon_tile(const StageArgs& A, const DevItem& it) {
     const DevBlock& B = A.blocks[it.block];
-    if (A.skip_dead && A.bad[B.case_id] < *A.step) return;
+    if (frozen_case(A, B)) return;
     const int c = (int)threadIdx.x >> 2, v = (int)threadIdx.x & 3;
     if (c >= it.r0) return;
     const int e = it.j0 + c;
@@ -1318,9 +1359,9 @@ __device__ __forceinline__ void ew_recon_tile(const StageArgs& A, const WorkItem
 }
 
 template <bool CART, int FLUX, bool GEN>
-__device__ __forceinline__ void ew_face_tile(const StageArgs& A, const WorkItem it) {
+__device__ __forceinline__ void ew_face_tile(const StageArgs& A, const DevItem& it) {
     const DevBlock& B = A.blocks[it.block];
-    if (A.skip_dead && A.bad[B.case_id] < *A.step) return;
+    if (frozen_case(A, B)) return;
     if ((int)threadIdx.x >= it.r0) return;
     const long long f = (long long)it.j0 + threadIdx.x;
     const phx::host::AdjBlock O{B.off / 4, B.foff};
@@ -1333,9 +1374,9 @@ __device__ __forceinline__ void ew_face_tile(const StageArgs& A, const WorkItem 
 }
 
 template <bool CART>
-__device__ __forceinline__ void ew_update_tile(const StageArgs& A, const WorkItem it) {
+__device__ __forceinline__ void ew_update_tile(const StageArgs& A, const DevItem& it) {
     const DevBlock& B = A.blocks[it.block];
-    if (A.skip_dead && A.bad[B.case_id] < *A.step) return;  // uniform over the workgroup
+    if (frozen_case(A, B)) return;  // uniform over the workgroup
     const int t = (int)threadIdx.x;
     double lane_dt = __longlong_as_double((long long)DT_INF_BITS);
     bool lane_bad = false;
@@ -1355,9 +1396,9 @@ __global__ void __launch_bounds__(EW_WG) k_ew_recon(StageArgs A) {
     int lo, hi, first, stride;
     item_range(A.nitems, lo, hi, first, stride);
     for (int i = first; i < hi; i += stride) {
-        const WorkItem it = ld_const(A.items, i);
+        const DevItem& it = const_ref(A.items, i);
         if (CK == 2) {  // items of both geometry kinds: the path of the item's block
-            if (A.blocks[it.block].kind == PHX_GEOM_CARTESIAN) ew_recon_tile<true, GEN>(A, it);
+            if (it.b.kind == PHX_GEOM_CARTESIAN) ew_recon_tile<true, GEN>(A, it);
             else ew_recon_tile<false, GEN>(A, it);
         } else {
             ew_recon_tile<CK == 1, GEN>(A, it);
@@ -1370,9 +1411,9 @@ __global__ void __launch_bounds__(EW_WG) k_ew_face(StageArgs A) {
     int lo, hi, first, stride;
     item_range(A.nitems, lo, hi, first, stride);
     for (int i = first; i < hi; i += stride) {
-        const WorkItem it = ld_const(A.items, i);
+        const DevItem& it = const_ref(A.items, i);
         if (CK == 2) {
-            if (A.blocks[it.block].kind == PHX_GEOM_CARTESIAN) ew_face_tile<true, FLUX, GEN>(A, it);
+            if (it.b.kind == PHX_GEOM_CARTESIAN) ew_face_tile<true, FLUX, GEN>(A, it);
             else ew_face_tile<false, FLUX, GEN>(A, it);
         } else {
             ew_face_tile<CK == 1, FLUX, GEN>(A, it);
@@ -1385,9 +1426,9 @@ __global__ void __launch_bounds__(EW_WG) k_ew_update(StageArgs A) {
     int lo, hi, first, stride;
     item_range(A.nitems, lo, hi, first, stride);
     for (int i = first; i < hi; i += stride) {
-        const WorkItem it = ld_const(A.items, i);
+        const DevItem& it = const_ref(A.items, i);
         if (CK == 2) {
-            if (A.blocks[it.block].kind == PHX_GEOM_CARTESIAN) ew_update_tile<true>(A, it);
+            if (it.b.kind == PHX_GEOM_CARTESIAN) ew_update_tile<true>(A, it);
             else ew_update_tile<false>(A, it);
         } else {
             ew_update_tile<CK == 1>(A, it);

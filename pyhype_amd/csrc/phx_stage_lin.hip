@@ -8,7 +8,9 @@ namespace {
 struct k_recon_x_lin_go {
     template <bool C, int F, int M, bool G>
     static void go(dim3 g, hipStream_t st, const StageArgs& A) {
-        constexpr int MM = G ? 3 : (M < 3 ? 3 : M);
+        // HLLL: 128 registers (4 waves per SIMD; 198.4 -> 195.4 us per step of 5 x 500^2 cells), Roe at
+        // least 134 (3 waves; 118.3 against 119.9 us on 8 x 150^2 cells)
+        constexpr int MM = G ? 3 : (F == 1 || M > 3 ? 4 : 3);
         hipLaunchKernelGGL((k_recon_x_lin<C ? 1 : 0, F, MM, G>), g, dim3(WAVE), 0, st, A);
     }
 };
