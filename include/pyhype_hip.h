@@ -237,9 +237,9 @@ int phx_step_vjp(phx_plan* plan, const double* stages, const double* dt_dev, dou
  * pyhype_amd/autotune.py.  No counterpart in the reference. */
 int phx_set_launch(phx_plan* plan, int32_t rows_per_item, int32_t grid_waves, int32_t waves_per_simd);
 
-/* Stage kernel variant: 0 = fused rolling rows (default; best for large meshes), 2 = fused with
- * workgroups of 4 waves that share their halo rows through LDS (rows_per_item rows per wave),
- * 1 = split into a
+/* Stage kernel variant: 0 = fused rolling rows (default; best for large meshes), 2 = one launch of
+ * workgroups that own a strip of 1 (rows_per_item 1) or 2 rows and share its states and faces through
+ * LDS, a wave per row and variable (best for meshes of about one workgroup per CU), 1 = split into a
  * reconstruction + x-face kernel, a y-face kernel and a residual + update kernel, which evaluates
  * every reconstruction and face flux exactly once (best for small meshes, where short fused items
  * spend most of their work on halo rows); rows_b = rows per work item of the update kernel

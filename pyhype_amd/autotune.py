@@ -88,10 +88,10 @@ def _time_steps(plan, steps: int) -> float:
 
 def candidates(rows: Sequence[int] = ROWS, grids: Sequence[int] = (0, 1024, 2048, 3072), waves: Sequence[int] = (2, 3),
                split_rows: Sequence[int] = (1, 2, 3, 4, 8), split_rows_b: Sequence[int] = (1, 2, 4, 8, 16, 32),
-               split_waves: Sequence[int] = (3, 4), shared_rows: Sequence[int] = (1, 2, 3, 4, 6),
+               split_waves: Sequence[int] = (3, 4), shared_rows: Sequence[int] = (1, 2),
                paired_rows: Sequence[int] = (1, 2, 3, 4, 6, 8, 12)):
     """The default search space: fused shapes (one workgroup per work item, grid 0, or a persistent
-    grid of `grids` workgroups that stride over the work list), shared-halo shapes (rows per wave),
+    grid of `grids` workgroups that stride over the work list), shared-halo shapes (rows per workgroup),
     split shapes, the element-wise stage, paired shapes (rows per item), and persistent grids of the
     split stages' kernels."""
     out = [{"variant": 0, "rows_per_item": r, "grid_waves": g, "waves_per_simd": w, "rows_b": 0}

@@ -350,7 +350,7 @@ int build_items(phx_plan* P) {
     const bool split = P->variant == 1 || P->variant >= 5;
     P->flat_q[0] = P->flat_q[1] = 0;
     const int strip = split ? STRIP_A : STRIP;
-    const int item_rows = P->variant == 2 ? WGW * rows : rows;  // shared-halo items: WGW waves of `rows`
+    const int item_rows = P->variant == 2 ? wg_rows(rows) : rows;  // shared-halo items: one row per inner wave
     for (int b = 0; b < P->nblocks; ++b) {
         const phx_block_desc& d = P->desc[b];
         const int kind = d.geom_kind == PHX_GEOM_CARTESIAN ? 1 : 0;
@@ -638,7 +638,7 @@ void launch_stage(phx_plan* P, StageArgs A, hipStream_t st) {
         return;
     }
     if (P->variant == 2) {
-        A.rows_wave = P->rows_per_item > 0 ? P->rows_per_item : 1;
+        A.rows_wave = wg_rows(P->rows_per_item);
         for_kinds(P, !P->items[0].empty(), !P->items[1].empty(), st, [&](int kind, hipStream_t s) {
             launch_kind<k_stage_wg_tag>(P, A, kind, P->ditems[kind], (int)P->items[kind].size(), P->grid[kind],
                                         2, s);

@@ -72,7 +72,7 @@ struct StageArgs {
     int* bad;          // per case: first step whose result was unrealizable (INT_MAX = none)
     const int* step;   // index of the step being computed (1-based)
     int skip_dead;     // skip the blocks of cases that failed at an earlier step
-    int rows_wave;     // shared-halo stage: rows per wave
+    int rows_wave;     // shared-halo and y-face stages: rows per workgroup
     double* sn;        // split stage: limited N and S states per cell (8 doubles, offset 2*off)
     double* p1;        // split stage: LW*(2 FW) - LE*(2 FE) per cell (4 doubles, state layout)
     double* yf;        // split stage: y-face fluxes (DevBlock::yoff)
@@ -345,159 +345,194 @@ __global__ void __launch_bounds__(WAVE, MINW) k_stage(StageArgs A) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// shared-halo stage: a workgroup of WGW waves takes WGW * rows_wave consecutive rows of one strip,
-// wave w the rows [a, b) = [r0 + w*rows_wave, ...).  Only the workgroup's outermost waves
-// reconstruct a halo row; the face between two waves of the workgroup is evaluated once, by the
-// upper wave, from the lower wave's last N state passed through LDS, and its flux is passed back.
-// Same arithmetic and association order as stage_item (the first and last rows of a wave complete
-// after the exchange).
+// shared-halo stage: one launch per stage for small meshes, where the time of a stage is the chain of one
+// wave, the latency of its loads and the instructions it runs for the first time (about 2 us of 10 went
+// into fetching them).  A workgroup takes R = 1 or 2 cell rows [r0, r1) of one strip with 4 (R + 2) waves:
+//   1. wave 4 i + v reconstructs variable v of row r0 - 1 + i (the outer two rows are halo) and writes
+//      the limited face states to LDS (the value itself beyond a block side);
+//   2. one wave per face row takes an x-face row or a y-face row from there, flux to LDS, while
+//   3. one wave per cell row loads what the update needs, and completes its row after the barrier.
+// A wave's chain is one variable's reconstruction, then one flux or one update, and every wave of a
+// phase runs the same code (one reconstruction, one flux), a third of the instructions of a wave that does
+// a whole row.  Compared with the split stage's two kernels it saves a launch (1 us between two kernels,
+// 2 until the first values have arrived) and the states and fluxes that pass through memory; the
+// price is (R + 2)/R of the reconstructions.  Same arithmetic and association order as stage_item.
 // ---------------------------------------------------------------------------------------------
-constexpr int WGW = 4;
+constexpr int WG_MAX_ROWS = 2;
+__host__ __device__ inline int wg_rows(int rows_per_item) { return rows_per_item > 1 ? WG_MAX_ROWS : 1; }
+constexpr int wg_waves(int rows) { return 4 * (rows + 2); }
 
-template <bool CART, int FLUX, bool GEN>
-__device__ __forceinline__ void stage_wg_item(const StageArgs& A, const DevItem& it, Q4* lds_N, Q4* lds_F) {
-    const DevBlock& B = A.blocks[it.block];
-    if (frozen_case(A, B)) return;  // uniform over the workgroup
+// doubles of LDS: E and W states of R rows, N and S of R + 1, x-fluxes of R rows, y-fluxes of R + 1
+constexpr int WG_PLANE = 4 * WAVE;
+constexpr int wg_lds(int rows) { return (6 * rows + 3) * WG_PLANE; }
+
+__device__ __forceinline__ double pick(const Q4& q, int v) {
+    return v == 0 ? q.v[0] : (v == 1 ? q.v[1] : (v == 2 ? q.v[2] : q.v[3]));
+}
+
+// Variable v of the stage state at row k of a wave's strip (k and v are the same for the whole wave, so
+// the row's place in the block is decided by scalar branches), in the reconstruction variables: cells at
+// the `inner` columns, ghost values beyond the south and north sides and, with GC in waves at a block
+// side (`edge`), at the two ghost columns.
+template <bool CART, bool GEN, bool GC>
+__device__ __forceinline__ double row_value(const StageArgs& A, const DevBlock& B, int k, int j, int v, bool inner,
+                                            bool edge) {
+    const bool inside = k >= 0 && k < B.ny;
+    const bool prim = GEN && A.ph.prim;
+    double x = 0.0;
+    if (inside && !prim && inner) x = gld(A.Uin, B.off + 4 * ((long)k * B.nx + j) + v);
+    if (!inside || prim || (GC && edge)) {
+        Q4 q = phx::q4zero();
+        bool full = false;
+        if (!inside) {
+            if (inner) q = k < 0 ? ghost_value<CART, PHX_S>(A.blocks, B, A.Uin, k, j) : ghost_value<CART, PHX_N>(A.blocks, B, A.Uin, k, j);
+            full = inner;
+        } else {
+            if (prim && inner) {
+                q = ld4(A.Uin + B.off + 4 * ((long)k * B.nx + j));
+                full = true;
+            }
+            if (GC && edge) {
+                if (j == -1) q = ghost_value<CART, PHX_W>(A.blocks, B, A.Uin, k, j);
+                if (j == B.nx) q = ghost_value<CART, PHX_E>(A.blocks, B, A.Uin, k, j);
+                full = full || j == -1 || j == B.nx;
+            }
+        }
+        if (prim) q = phx::prim_q4(phx::cons_to_prim(q, A.ph));
+        if (full) x = pick(q, v);
+    }
+    return x;
+}
+
+template <bool CART, int FLUX, int R, bool GEN>
+__device__ __forceinline__ void stage_wg_item(const StageArgs& A, const DevItem& it, double* lds) {
+    const DevBlock B = it.b;  // in scalar registers
     const int lane = threadIdx.x & (WAVE - 1);
-    const int w = threadIdx.x / WAVE;
-    const int nx = B.nx, ny = B.ny;
-    const int R = A.rows_wave;
-    const int a = it.r0 + w * R, b = min(a + R, it.r1);
-    const int wtop = (it.r1 - it.r0 - 1) / R;
-    const bool active = a < it.r1;
-    const bool bottom = (w == 0), top = (w == wtop);
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
+    const int nx = B.nx, ny = B.ny, nrow = it.r1 - it.r0;  // (the last item of a strip may be shorter)
     const int j = it.j0 - HALO + lane;
-    const bool valid = (j >= -1) && (j <= nx);
     const bool inner = (j >= 0) && (j < nx);
-    const bool gcol = (j == -1) || (j == nx);
-    const bool recon = inner && (j >= it.j0 - 1) && (j <= it.j0 + STRIP);
-    const bool xface = (j >= it.j0) && (j <= min(it.j0 + STRIP, nx));
     const bool owner = inner && (j >= it.j0) && (j < it.j0 + STRIP);
-    const double dt = (A.dt != nullptr) ? ld_const(A.dt, B.case_id) : 0.0;
-    const Phys ph = A.ph;
+    const bool west = it.j0 == 0, east = it.j0 + STRIP + HALO > nx;  // strips that touch the block's sides
+    double* const sE = lds;                                // [R][4][WAVE]: face states of row r0 + i
+    double* const sW = sE + R * WG_PLANE;
+    double* const sN = sW + R * WG_PLANE;                  // [R + 1]: N states of row r0 - 1 + i
+    double* const sS = sN + (R + 1) * WG_PLANE;            // [R + 1]: S states of row r0 + i
+    double* const fX = sS + (R + 1) * WG_PLANE;            // [R]: x-fluxes of row r0 + i
+    double* const fY = fX + R * WG_PLANE;                  // [R + 1]: y-fluxes of face row r0 + i
 
+    {   // one variable of one row
+        const int i = w >> 2, v = w & 3, k = it.r0 - 1 + i;
+        const bool used = i <= nrow + 1;
+        const bool real = used && k >= 0 && k < ny;
+        const bool recon = real && inner && (j >= it.j0 - 1) && (j <= it.j0 + STRIP);
+        double c = 0.0, m = 0.0, p = 0.0;
+        phx::CellGeo g;
+        if (used) c = row_value<CART, GEN, true>(A, B, k, j, v, inner, west || east);
+        if (real) {
+            m = row_value<CART, GEN, false>(A, B, k - 1, j, v, inner, false);
+            p = row_value<CART, GEN, false>(A, B, k + 1, j, v, inner, false);
+            if (recon) g = cell_geo<CART>(B, k, j);
+        }
+        // a frozen case leaves here (uniform over the workgroup; nothing has been written)
+        if (frozen_case(A, B)) return;
+        const double e = __shfl_down(c, 1, WAVE), we = __shfl_up(c, 1, WAVE);
+        double qE = c, qW = c, qN = c, qS = c;
+        if (recon) phx::reconstruct_var<GEN>(c, we, e, m, p, g, A.ph.limiter, qE, qW, qN, qS);
+        const int at = v * WAVE + lane;
+        if (i >= 1 && i <= nrow) {
+            sE[(i - 1) * WG_PLANE + at] = qE;
+            sW[(i - 1) * WG_PLANE + at] = qW;
+        }
+        if (i <= nrow) sN[i * WG_PLANE + at] = qN;
+        if (i >= 1 && used) sS[(i - 1) * WG_PLANE + at] = qS;
+    }
+    constexpr int WAVES = wg_waves(R);
+    const int u = w - (WAVES - R);  // the last R waves: update of row r0 + u
+    if (u < 0) {
+        // x-face row w (w < nrow) or y-face row w - nrow (up to nrow)
+        const bool xdir = w < nrow;
+        const int y = w - nrow;
+        const bool task = y <= nrow;
+        const int k = xdir ? it.r0 + w : it.r0 + y;
+        const bool on = task && (xdir ? (j >= it.j0) && (j <= min(it.j0 + STRIP, nx)) : owner);
+        double cs = 1.0, sn = 0.0;
+        if (!CART && on) {
+            const GenG G{B.geom, nx, ny};
+            cs = xdir ? G.V(F_c, k, j) : G.H(F_c, k, j);
+            sn = xdir ? G.V(F_s, k, j) : G.H(F_s, k, j);
+        }
+        __syncthreads();
+        if (on) {
+            const double* const pl = xdir ? sE + w * WG_PLANE + lane - 1 : sN + y * WG_PLANE + lane;
+            const double* const pr = xdir ? sW + w * WG_PLANE + lane : sS + y * WG_PLANE + lane;
+            Q4 L, Rs;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                L.v[c] = pl[c * WAVE];
+                Rs.v[c] = pr[c * WAVE];
+            }
+            // beyond a side the slot holds the ghost value (outer_state's)
+            if (xdir) {
+                if (west && j == 0) L = outer_state<CART>(B, PHX_W, Rs, L, k, j);
+                if (east && j == nx) Rs = outer_state<CART>(B, PHX_E, L, Rs, k, j);
+            } else {
+                if (k == 0) L = outer_state<CART>(B, PHX_S, Rs, L, k, j);
+                if (k == ny) Rs = outer_state<CART>(B, PHX_N, L, Rs, k - 1, j);
+            }
+            if (!CART) {
+                L = phx::rotate(L, cs, sn);
+                Rs = phx::rotate(Rs, cs, sn);
+            } else if (!xdir) {
+                L = phx::rotate90(L);
+                Rs = phx::rotate90(Rs);
+            }
+            Q4 F = flux_of<FLUX, GEN>(L, Rs, A.ph);
+            if (!CART) F = phx::unrotate(F, cs, sn);
+            else if (!xdir) F = phx::unrotate90(F);
+            double* const pf = (xdir ? fX + w * WG_PLANE : fY + y * WG_PLANE) + lane;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) pf[c * WAVE] = F.v[c];
+        }
+        __syncthreads();
+        return;
+    }
+    __syncthreads();
+    const bool row = u < nrow;
+    const int k = it.r0 + u;
+    Q4 pre[EMIT_CHUNK];
+    double LW = 0.0, LE = 0.0, LS = 0.0, LN = 0.0, Ac = 1.0, dxc = 0.0;
+    const double dt = (A.dt != nullptr) ? ld_const(A.dt, B.case_id) : 0.0;
+    if (row && owner) {
+        cell_L<CART>(B, k, j, LW, LE, LS, LN, Ac);
+        prefetch_sources(A, B, k, j, pre);
+        if (CART && A.dtmin != nullptr) dxc = CartGT<true>{B.geom, nx, ny}.col(C_dx, j);
+    }
+    __syncthreads();
+    if (!row) return;
     double lane_dt = __longlong_as_double((long long)DT_INF_BITS);
     bool lane_bad = false;
-    // first row of a wave above the bottom: its S face waits for the exchange
-    Q4 first_S = phx::q4zero(), first_part = phx::q4zero(), first_FN = phx::q4zero();
-    double first_LS = 0.0, first_LN = 0.0, first_A = 1.0;
-    // last row of a wave below the top: its N face waits for the exchange
-    Q4 part = phx::q4zero(), QNprev = phx::q4zero();
-    double prevLN = 0.0, prevA = 1.0;
-
-    if (active) {
-        const int kr0 = bottom ? max(a - 1, 0) : a;
-        const int kr1 = top ? min(it.r1, ny) : b - 1;
-        Q4 Um = phx::q4zero(), Uc = phx::q4zero(), Up = phx::q4zero();
-        if (inner) Um = fetch_r<CART, GEN>(A.blocks, B, A.Uin, kr0 - 1, j, ph);
-        if (valid) Uc = fetch_r<CART, GEN>(A.blocks, B, A.Uin, kr0, j, ph);
-        for (int k = kr0; k <= kr1; ++k) {
-            const bool real = (k < ny);
-            if (real) {
-                if (inner) Up = fetch_r<CART, GEN>(A.blocks, B, A.Uin, k + 1, j, ph);
-                else if (gcol && k + 1 <= kr1 && k + 1 < ny) Up = fetch_r<CART, GEN>(A.blocks, B, A.Uin, k + 1, j, ph);
-            }
-            const Q4 Uw = shfl_up1(Uc);
-            const Q4 Ue = shfl_down1(Uc);
-            phx::Recon r;
-            r.E = r.W = r.N = r.S = phx::q4zero();
-            if (real && recon) {
-                const phx::CellGeo g = cell_geo<CART>(B, k, j);
-                r = phx::reconstruct<GEN>(Uc, Uw, Ue, Um, Up, g, ph.limiter);
-            }
-            const Q4 qsend = (j == -1) ? Uc : r.E;
-            const Q4 QEl = shfl_up1(qsend);
-            const bool xrow = (k >= a) && (k < b);
-            Q4 FW = phx::q4zero();
-            if (xrow && xface) {
-                const Q4 L = (j == 0) ? outer_state<CART>(B, PHX_W, r.W, QEl, k, j) : QEl;
-                const Q4 R2 = (j == nx) ? outer_state<CART>(B, PHX_E, QEl, Uc, k, j) : r.W;
-                FW = xflux<CART, FLUX, GEN>(B, L, R2, k, j, ph);
-            }
-            const Q4 FE = shfl_down1(FW);
-            if (k >= a && owner) {
-                const bool defer_S = (k == a) && !bottom;
-                Q4 F = phx::q4zero();
-                if (!defer_S) {
-                    const Q4 L = (k == 0) ? outer_state<CART>(B, PHX_S, r.S, Um, k, j) : QNprev;
-                    const Q4 R2 = (k == ny) ? outer_state<CART>(B, PHX_N, QNprev, Uc, k - 1, j) : r.S;
-                    F = yflux<CART, FLUX, GEN>(B, L, R2, k, j, ph);
-                    if (k - 1 >= a) {
-                        if (k - 1 == a && !bottom) {
-                            first_FN = F;
-                        } else {
-                            Q4 Res;
+    if (owner) {
+        Q4 Res;
 #pragma unroll
-                            for (int c = 0; c < 4; ++c) Res.v[c] = 0.5 * (part.v[c] - prevLN * (2.0 * F.v[c]));
-                            phx::div_all(Res.v, prevA, Res.v);
-                            emit_row<CART>(A, B, k - 1, j, dt, Res, lane_dt, lane_bad);
-                        }
-                    }
-                }
-                if (xrow) {
-                    double LW, LE, LS, LN, Ac;
-                    cell_L<CART>(B, k, j, LW, LE, LS, LN, Ac);
-                    if (defer_S) {
-#pragma unroll
-                        for (int c = 0; c < 4; ++c) first_part.v[c] = LW * (2.0 * FW.v[c]) - LE * (2.0 * FE.v[c]);
-                        first_S = r.S;
-                        first_LS = LS;
-                        first_LN = LN;
-                        first_A = Ac;
-                    } else {
-#pragma unroll
-                        for (int c = 0; c < 4; ++c)
-                            part.v[c] = (LW * (2.0 * FW.v[c]) - LE * (2.0 * FE.v[c])) + LS * (2.0 * F.v[c]);
-                    }
-                    prevLN = LN;
-                    prevA = Ac;
-                }
-            }
-            QNprev = r.N;
-            Um = Uc;
-            Uc = Up;
+        for (int c = 0; c < 4; ++c) {
+            const double FW = fX[u * WG_PLANE + c * WAVE + lane], FE = fX[u * WG_PLANE + c * WAVE + lane + 1];
+            const double FS = fY[u * WG_PLANE + c * WAVE + lane], FN = fY[(u + 1) * WG_PLANE + c * WAVE + lane];
+            Res.v[c] = 0.5 * (((LW * (2.0 * FW) - LE * (2.0 * FE)) + LS * (2.0 * FS)) - LN * (2.0 * FN));
         }
-        if (!top && owner) lds_N[w * WAVE + lane] = QNprev;  // N state of row b-1
-    }
-    __syncthreads();
-    Q4 FS_first = phx::q4zero();
-    if (active && !bottom && owner) {
-        // face between a-1 (last row of wave w-1) and a
-        FS_first = yflux<CART, FLUX, GEN>(B, lds_N[(w - 1) * WAVE + lane], first_S, a, j, ph);
-        lds_F[w * WAVE + lane] = FS_first;
-    }
-    __syncthreads();
-    if (active && owner) {
-        const bool single = (b - 1 == a);
-        if (!bottom) {
-            const Q4 FN = (single && !top) ? lds_F[(w + 1) * WAVE + lane] : first_FN;
-            Q4 Res;
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
-                Res.v[c] = 0.5 * ((first_part.v[c] + first_LS * (2.0 * FS_first.v[c])) - first_LN * (2.0 * FN.v[c]));
-            phx::div_all(Res.v, first_A, Res.v);
-            emit_row<CART>(A, B, a, j, dt, Res, lane_dt, lane_bad);
-        }
-        if (!top && !(single && !bottom)) {
-            const Q4 FN = lds_F[(w + 1) * WAVE + lane];
-            Q4 Res;
-#pragma unroll
-            for (int c = 0; c < 4; ++c) Res.v[c] = 0.5 * (part.v[c] - prevLN * (2.0 * FN.v[c]));
-            phx::div_all(Res.v, prevA, Res.v);
-            emit_row<CART>(A, B, b - 1, j, dt, Res, lane_dt, lane_bad);
-        }
+        phx::div_all(Res.v, Ac, Res.v);
+        emit_row<CART, true>(A, B, k, j, dt, Res, lane_dt, lane_bad, pre, dxc);
     }
     reduce_item(A, B, lane, lane_dt, lane_bad);
 }
 
-template <bool CART, int FLUX, int MINW, bool GEN>
-__global__ void __launch_bounds__(WGW * WAVE, MINW) k_stage_wg(StageArgs A) {
-    __shared__ Q4 lds_N[WGW * WAVE];
-    __shared__ Q4 lds_F[WGW * WAVE];
+template <bool CART, int FLUX, int R, bool GEN>
+__global__ void __launch_bounds__(wg_waves(R) * WAVE) k_stage_wg(StageArgs A) {
+    __shared__ double lds[wg_lds(R)];
     int lo, hi, first, stride;
     item_range(A.nitems, lo, hi, first, stride);
     for (int i = first; i < hi; i += stride) {
-        stage_wg_item<CART, FLUX, GEN>(A, const_ref(A.items, i), lds_N, lds_F);
+        stage_wg_item<CART, FLUX, R, GEN>(A, const_ref(A.items, i), lds);
         __syncthreads();  // the next item reuses the exchange buffers
     }
 }

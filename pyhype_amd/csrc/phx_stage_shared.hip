@@ -8,7 +8,8 @@ namespace {
 struct k_stage_wg_go {
     template <bool C, int F, int M, bool G>
     static void go(dim3 g, hipStream_t st, const StageArgs& A) {
-        hipLaunchKernelGGL((k_stage_wg<C, F, 2, G>), g, dim3(WGW * WAVE), 0, st, A);
+        if (A.rows_wave == 1) hipLaunchKernelGGL((k_stage_wg<C, F, 1, G>), g, dim3(wg_waves(1) * WAVE), 0, st, A);
+        else hipLaunchKernelGGL((k_stage_wg<C, F, 2, G>), g, dim3(wg_waves(2) * WAVE), 0, st, A);
     }
 };
 struct k_stage_pair_go {
