@@ -79,9 +79,52 @@ def validate_config(config) -> List[List[float]]:
     return butcher_table(config.time_integrator, config)
 
 
+# Launch shape of a workload without a tuned one (us per RK stage measured on an MI355X, 256 CUs, smooth
+# flow, the alternatives beside it):
+#  * The shared-halo stage (variant 2) while its workgroups, one per CU, fit about one and a half rounds
+#    of the chip: with one row each up to 256 workgroups (64^2: 11.0 against 14.6 with the split
+#    stage and 25.7 fused; 8 x 32^2: 11.1 against 15.9), with two rows up to 384 (128^2, 192 of them:
+#    11.7 against 14.9; six 93 x 61 HLLL blocks, 372: 25.5 against 32.4).  At 500 it falls behind (5 x
+#    100^2 HLLL: 26.3 against 22.5).  A mesh of both geometry kinds takes two launches of it, the
+#    split stage one per kernel over both (4 x 50^2: 29.2 against 22.5).
+#  * The split stage with one y-face per wave up to the size where the states that pass between its
+#    kernels no longer stay in the caches: strips (variant 6) while a Cartesian mesh has fewer than 10^5
+#    cells (256^2: 18.2 against 20.4), row-major (variant 7) beyond (400^2: 26.6 against 27.4;
+#    8 x 150^2: 29.5 against 33.8), up to 10^6 cells with Roe (1.1 x 10^6: 98 against 96 fused;
+#    2.25 x 10^6: 220 against 167) and 2.5 x 10^6 with HLLL, whose fused kernel is bound by its
+#    registers (1.1 x 10^6: 120 against 136; 2.8 x 10^6: 319 against 326).
+#    From 2.5 x 10^5 cells the work lists are dealt to the XCDs in chunks of 64 items, so that the faces
+#    of neighbouring rows meet in one L2 (8 x 10^5: 94.1 against 99.6).
+#  * The fused stage beyond, with items of 8 rows or more (1.1 x 10^6 cells: 4 rows 111.9, 8 rows 96.2;
+#    2.4 x 10^6: 4 rows 221.6, 10 rows 201.0).
+SHARED_ITEMS = (256, 384)          # workgroups of the shared-halo stage with 1 and 2 rows
+STRIP_CELLS = 100_000
+DEALT_CELLS = 250_000
+SPLIT_CELLS = {"Roe": 1_000_000, "HLLL": 2_500_000}
+FUSED_ROWS = 8
+
+
 def default_rows(cells: int) -> int:
-    """Rows per work item when no tuned value is cached: about 4096 items of 60 columns."""
+    """Rows per item of the fused stage: about 4096 items of 60 columns."""
     return int(max(2, min(64, round(cells / (60 * 4096)))))
+
+
+def default_shape(plan) -> dict:
+    """``DevicePlan.set_launch`` arguments for a workload without a tuned shape (see above)."""
+    cells = plan.cells()
+    if plan.quadrature_points > 1:   # the split stage of the plan; rows of a reconstruction item
+        return {"rows_per_item": 1 if cells < STRIP_CELLS else 2}
+    kinds = {e.cartesian for e in plan.blocks}
+    strips = [(-(-e.nx // 60), e.ny) for e in plan.blocks]
+    for rows, most in zip((1, 2), SHARED_ITEMS):
+        if len(kinds) == 1 and sum(n * -(-ny // rows) for n, ny in strips) <= most:
+            return {"rows_per_item": rows, "variant": 2}
+    if cells > SPLIT_CELLS[plan.flux]:
+        return {"rows_per_item": max(FUSED_ROWS, default_rows(cells))}
+    if cells < STRIP_CELLS and kinds != {False}:
+        return {"rows_per_item": 1, "waves_per_simd": 3, "variant": 6, "rows_b": 1}
+    return {"rows_per_item": 1, "waves_per_simd": 3, "variant": 7, "rows_b": 3,
+            "xcd_chunk": 64 if cells > DEALT_CELLS else 0}
 
 
 def mesh_dict(mesh_config) -> Dict[int, dict]:
@@ -143,7 +186,9 @@ class Euler2DBatch:
 
             self.tuned = use_tuning_cache and autotune.apply_cached(self.plan)
             if not self.tuned:
-                self.plan.set_launch(default_rows(self.plan.cells()), grid_waves)
+                # a persistent grid is asked for: the fused stage strides over its list with it
+                shape = {"rows_per_item": default_rows(self.plan.cells())} if grid_waves else default_shape(self.plan)
+                self.plan.set_launch(grid_waves=grid_waves, **shape)
         self.case_blocks: List[Dict[int, HostBlock]] = []
         for c, entries in enumerate(self.plan.case_blocks):
             self.case_blocks.append({n: HostBlock(self.configs[c], e) for n, e in entries.items()})
