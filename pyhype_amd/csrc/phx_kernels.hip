@@ -19,7 +19,8 @@ using namespace phx::stage;
 
 namespace {
 
-constexpr int GRAPH_STEPS = 8;  // steps captured in the multi-step graph of phx_run
+// Step graphs of phx_run: graph g holds 2^g steps.
+constexpr int GRAPHS = phx_plan::GRAPHS;
 int dt_slots_for(int ncases) {
     int n = DT_SLOTS;
     while (n > 4 && (long)n * ncases > 256) n >>= 1;
@@ -114,11 +115,11 @@ __global__ void __launch_bounds__(FIN_THREADS) k_finalize(int ncases, int nslot,
 }
 __global__ void k_reset(int ncases, int nslot, const double* t0, double* t, unsigned long long* dtmin, int* bad,
                         int* step, int step0) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;  // one thread per (case, slot)
-    if (c < ncases * nslot) dtmin[(long)c * DT_STRIDE] = DT_INF_BITS;
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;  // one thread per (set, case, slot)
+    if (c < 2 * ncases * nslot) dtmin[(long)c * DT_STRIDE] = DT_INF_BITS;
     if (c < ncases) {
         t[c] = t0[c];
-        bad[c] = 0x7fffffff;
+        bad[c] = NEVER;
     }
     if (c == 0) step[0] = step0;
 }
@@ -443,7 +444,7 @@ int build_items(phx_plan* P) {
 
 // Destroys the captured step graphs (they hold the launch list and the state pointer).
 void release_graphs(phx_plan* P) {
-    for (int g = 0; g < 2; ++g) {
+    for (int g = 0; g < GRAPHS; ++g) {
         if (P->gexec[g]) { (void)hipGraphExecDestroy(P->gexec[g]); P->gexec[g] = nullptr; }
         if (P->graph[g]) { (void)hipGraphDestroy(P->graph[g]); P->graph[g] = nullptr; }
     }
@@ -466,11 +467,13 @@ StageArgs base_args(phx_plan* P) {
 // one launch of kernel family T over the items of one geometry kind; minw = register budget in
 // waves per SIMD (2, 3 or 4)
 template <class T>
-void launch_kind(const phx_plan* P, StageArgs A, int kind, const DevItem* items, int nitems, int grid, int minw,
+void launch_kind(const phx_plan* P, StageArgs& S, int kind, const DevItem* items, int nitems, int grid, int minw,
                  hipStream_t st) {
+    StageArgs A = S;
     A.items = items;
     A.nitems = nitems;
-    T::launch(P, kind, minw, dim3(grid), st, A);
+    T::launch(P, kind, minw, dim3(grid + A.fold_blocks), st, A);
+    S.fold_blocks = 0;  // the stage's first launch takes the extra workgroups
 }
 
 // One phase of a stage over both geometry kinds: launch(kind, stream) for each kind that has work.
@@ -516,7 +519,7 @@ void launch_stage(phx_plan* P, StageArgs A, hipStream_t st) {
         A.sn = P->sn;
         A.p1 = P->p1;
         A.rows_wave = std::min(std::max(P->rows_b, 1), YU_MAX_ROWS);
-        if (P->ditems_m[2]) launch_recon_x_lin_mixed(P, A, st);
+        if (P->ditems_m[2]) launch_recon_x_lin_mixed(P, A, st);  // (takes A.fold_blocks; the others ignore them)
         else
             for_kinds(P, !P->items_f[0].empty(), !P->items_f[1].empty(), st, [&](int kind, hipStream_t s) {
                 launch_kind<k_recon_x_lin_tag>(P, A, kind, P->ditems_f[kind], (int)P->items_f[kind].size(),
@@ -653,8 +656,8 @@ void launch_stage(phx_plan* P, StageArgs A, hipStream_t st) {
 }
 
 void launch_dt_reduce(phx_plan* P, const double* U, hipStream_t st) {
-    hipLaunchKernelGGL(k_fill_inf, dim3((P->ncases * P->nslot + 255) / 256), dim3(256), 0, st, P->ncases, P->nslot,
-                       P->dtmin);
+    const int sets = 2 * P->ncases;  // both sets of the minima
+    hipLaunchKernelGGL(k_fill_inf, dim3((sets * P->nslot + 255) / 256), dim3(256), 0, st, sets, P->nslot, P->dtmin);
     for (int kind = 0; kind < 2; ++kind) {
         const int n = (int)P->items[kind].size();
         if (!n) continue;
@@ -679,9 +682,46 @@ double* map_buf(phx_plan* P, const BufMap& M, int id, bool write) {
     return P->acc[id - BUF_ACC0];
 }
 
-void launch_prog_stage_mapped(phx_plan* P, size_t s, const BufMap& M, hipStream_t st) {
+// CFL minima a step reads (set = its parity in the run) or writes (the other set)
+unsigned long long* dtmin_set(const phx_plan* P, int set) {
+    return P->dtmin + (size_t)(set & 1) * P->ncases * P->nslot * DT_STRIDE;
+}
+
+// Whether a step's kernels take the closing of the step before along (StepFold).  The fused and paired
+// stages do not: they run meshes whose steps take 100 times as long.
+bool folds(const phx_plan* P) {
+    return P->variant == 2 ? P->progs.size() > 1 : P->variant != 0 && P->variant != 4;
+}
+
+// dt, times and counter of the next step as a kernel, where the step's own kernels do not take it along
+void open_step(phx_plan* P, int parity, const double* frozen, hipStream_t st) {
+    if (folds(P)) return;
+    hipLaunchKernelGGL(k_finalize, dim3(1), dim3(FIN_THREADS), 0, st, P->ncases, P->nslot, P->ph.cfl,
+                       dtmin_set(P, parity), P->tfinal, P->t, P->dt, P->step, P->bad, frozen, 1);
+}
+
+// What stage s of a step takes along; parity as in open_step
+void fold_step_into(const phx_plan* P, StageArgs& A, size_t s, int parity, const double* frozen) {
+    if (!folds(P) || s > (P->variant == 2 ? 1 : 0)) return;
+    A.fold_mode = P->variant != 2 ? FOLD_ALL : (s == 0 ? FOLD_DT : FOLD_TIME);
+    A.fold_set = parity & 1;
+    A.fold_blocks = (P->ncases * P->nslot + WAVE - 1) / WAVE;
+    A.fold = P->fold;
+    A.frozen = frozen;
+}
+
+// A stage's place in a step: the step's number in the run (its parity counts) and its schedule
+struct InStep {
+    int number;
+    const double* frozen;
+};
+
+// step: null for a stage on its own, which takes nothing along
+void launch_prog_stage_mapped(phx_plan* P, size_t s, const BufMap& M, hipStream_t st,
+                              const InStep* step) {
     const StageProg& g = P->progs[s];
     StageArgs A = base_args(P);
+    if (step) fold_step_into(P, A, s, step->number, step->frozen);
     A.Uin = map_buf(P, M, g.in, false);
     A.nout = (int)g.outs.size();
     for (int m = 0; m < A.nout; ++m) {
@@ -691,23 +731,25 @@ void launch_prog_stage_mapped(phx_plan* P, size_t s, const BufMap& M, hipStream_
     }
     A.state_out = g.state_out;
     A.skip_dead = 1;
-    if (g.state_out >= 0) A.dtmin = P->dtmin;
+    if (g.state_out >= 0) A.dtmin = dtmin_set(P, step ? step->number + 1 : 1);
     launch_stage(P, A, st);
 }
 
-void launch_prog_stage(phx_plan* P, double* U, size_t s, hipStream_t st) {
+void launch_prog_stage(phx_plan* P, double* U, size_t s, hipStream_t st,
+                       const InStep* step = nullptr) {
     const StageProg& g = P->progs[s];
     int sw = BUF_S0;
     for (const StageOut& o : g.outs)
         if (o.dst == BUF_S0 || o.dst == BUF_S1) sw = o.dst;
     const BufMap M{U, U, buf_ptr(P, U, g.in == BUF_USER ? BUF_S0 : g.in), buf_ptr(P, U, sw)};
-    launch_prog_stage_mapped(P, s, M, st);
+    launch_prog_stage_mapped(P, s, M, st, step);
 }
 
-void launch_step(phx_plan* P, double* U, hipStream_t st, const double* frozen) {
-    hipLaunchKernelGGL(k_finalize, dim3(1), dim3(FIN_THREADS), 0, st, P->ncases, P->nslot, P->ph.cfl, P->dtmin, P->tfinal, P->t,
-                       P->dt, P->step, P->bad, frozen, 1);
-    for (size_t s = 0; s < P->progs.size(); ++s) launch_prog_stage(P, U, s, st);
+// one step, the number-th of its run (from launch_dt_reduce, or with a schedule)
+void launch_step(phx_plan* P, double* U, hipStream_t st, const double* frozen, int number) {
+    open_step(P, number, frozen, st);
+    const InStep step{number, frozen};
+    for (size_t s = 0; s < P->progs.size(); ++s) launch_prog_stage(P, U, s, st, &step);
     if (P->copy_back)
         (void)hipMemcpyAsync(U, P->sbuf[0], (size_t)P->state_len * sizeof(double), hipMemcpyDeviceToDevice, st);
 }
@@ -736,7 +778,7 @@ int phx_plan_destroy(phx_plan* P) {
                     P->ditems_e[1][0], P->ditems_e[1][1], P->ditems_e[2][0], P->ditems_e[2][1],
                     P->ditems_em[0], P->ditems_em[1], P->ditems_em[2], P->ditems_m[0], P->ditems_m[1],
                     P->ditems_m[2],
-                    P->sbuf[0], P->sbuf[1], P->dt, P->t, P->tfinal, P->dtmin, P->step, P->bad, P->dghost_off};
+                    P->sbuf[0], P->sbuf[1], P->dt, P->t, P->tfinal, P->dtmin, P->step, P->bad, P->fold, P->dghost_off};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (int m = 0; m < MAX_ACC; ++m)
@@ -880,16 +922,19 @@ int phx_plan_create(const phx_plan_desc* D, phx_plan** out) {
     PHX_CKP(hipMalloc(&P->dt, cb));
     PHX_CKP(hipMalloc(&P->t, cb));
     PHX_CKP(hipMalloc(&P->tfinal, cb));
-    PHX_CKP(hipMalloc(&P->dtmin, (size_t)D->ncases * P->nslot * DT_STRIDE * sizeof(unsigned long long)));
+    PHX_CKP(hipMalloc(&P->dtmin, (size_t)2 * D->ncases * P->nslot * DT_STRIDE * sizeof(unsigned long long)));
     PHX_CKP(hipMalloc(&P->step, sizeof(int)));
     PHX_CKP(hipMalloc(&P->bad, D->ncases * sizeof(int)));
+    const StepFold fold{P->ncases, P->ph.cfl, P->dtmin, P->tfinal, P->t, P->dt, P->step};
+    PHX_CKP(hipMalloc(&P->fold, sizeof(fold)));
+    PHX_CKP(hipMemcpy(P->fold, &fold, sizeof(fold), hipMemcpyHostToDevice));
     PHX_CKP(hipMemcpy(P->tfinal, D->t_final, cb, hipMemcpyHostToDevice));
     PHX_CKP(hipMemset(P->dt, 0, cb));
     std::vector<double> zeros(D->ncases, 0.0);
     double* t0 = nullptr;
     PHX_CKP(hipMalloc(&t0, cb));
     PHX_CKP(hipMemcpy(t0, zeros.data(), cb, hipMemcpyHostToDevice));
-    hipLaunchKernelGGL(k_reset, dim3((D->ncases * P->nslot + 255) / 256), dim3(256), 0, 0, D->ncases, P->nslot, t0, P->t,
+    hipLaunchKernelGGL(k_reset, dim3((2 * D->ncases * P->nslot + 255) / 256), dim3(256), 0, 0, D->ncases, P->nslot, t0, P->t,
                        P->dtmin,
                        P->bad, P->step, 0);
     PHX_CKP(hipGetLastError());
@@ -915,7 +960,7 @@ int phx_reset(phx_plan* P, const double* t0_host, int32_t step0, void* stream) {
     double* t0 = nullptr;
     PHX_CK(hipMalloc(&t0, cb));
     PHX_CK(hipMemcpy(t0, t0_host, cb, hipMemcpyHostToDevice));
-    hipLaunchKernelGGL(k_reset, dim3((P->ncases * P->nslot + 255) / 256), dim3(256), 0, st, P->ncases, P->nslot, t0,
+    hipLaunchKernelGGL(k_reset, dim3((2 * P->ncases * P->nslot + 255) / 256), dim3(256), 0, st, P->ncases, P->nslot, t0,
                        P->t, P->dtmin,
                        P->bad, P->step, step0);
     PHX_CK(hipGetLastError());
@@ -931,26 +976,28 @@ int phx_run(phx_plan* P, double* U, int32_t nsteps, int32_t use_graph, void* str
     launch_dt_reduce(P, U, st);
     PHX_CK(hipGetLastError());
     if (!use_graph) {
-        for (int s = 0; s < nsteps; ++s) launch_step(P, U, st, nullptr);
+        for (int s = 0; s < nsteps; ++s) launch_step(P, U, st, nullptr, s);
         PHX_CK(hipGetLastError());
         return PHX_OK;
     }
     if (P->graph_U != U) release_graphs(P);
-    // GRAPH_STEPS steps per replay while enough remain (one graph launch per GRAPH_STEPS steps),
-    // then single steps
-    const int ng = nsteps / GRAPH_STEPS, n1 = nsteps % GRAPH_STEPS;
-    for (int g = 0; g < 2; ++g) {  // both captured on first use, so that later calls only replay
-        if (P->gexec[g]) continue;
+    // The largest graph while enough steps remain, then one graph for each bit of the rest, largest
+    // first: every graph but the last starts after an even number of steps, so that one capture of each
+    // size fits the alternation of the minima.  Captured when first needed; later calls replay.
+    const int most = 1 << (GRAPHS - 1);
+    for (int g = 0; g < GRAPHS; ++g) {
+        if (P->gexec[g] || !(g == GRAPHS - 1 ? nsteps >= most : (nsteps >> g) & 1)) continue;
         PHX_CK(hipStreamBeginCapture(P->cap_stream, hipStreamCaptureModeThreadLocal));
-        for (int s = 0; s < (g == 0 ? 1 : GRAPH_STEPS); ++s) launch_step(P, U, P->cap_stream, nullptr);
+        for (int s = 0; s < 1 << g; ++s) launch_step(P, U, P->cap_stream, nullptr, s);
         PHX_CK(hipStreamEndCapture(P->cap_stream, &P->graph[g]));
         PHX_CK(hipGraphInstantiate(&P->gexec[g], P->graph[g], nullptr, nullptr, 0));
     }
     P->graph_U = U;
     PHX_CK(hipEventRecord(P->ev_a, st));
     PHX_CK(hipStreamWaitEvent(P->cap_stream, P->ev_a, 0));
-    for (int s = 0; s < ng; ++s) PHX_CK(hipGraphLaunch(P->gexec[1], P->cap_stream));
-    for (int s = 0; s < n1; ++s) PHX_CK(hipGraphLaunch(P->gexec[0], P->cap_stream));
+    for (int s = 0; s < nsteps / most; ++s) PHX_CK(hipGraphLaunch(P->gexec[GRAPHS - 1], P->cap_stream));
+    for (int g = GRAPHS - 2; g >= 0; --g)
+        if ((nsteps >> g) & 1) PHX_CK(hipGraphLaunch(P->gexec[g], P->cap_stream));
     PHX_CK(hipEventRecord(P->ev_b, P->cap_stream));
     PHX_CK(hipStreamWaitEvent(st, P->ev_b, 0));
     return PHX_OK;
@@ -959,7 +1006,7 @@ int phx_run(phx_plan* P, double* U, int32_t nsteps, int32_t use_graph, void* str
 int phx_run_frozen(phx_plan* P, double* U, int32_t nsteps, const double* dt_sched, void* stream) {
     if (!P || !U || (!dt_sched && nsteps > 0)) return fail(PHX_E_INVALID, "null argument");
     hipStream_t st = (hipStream_t)stream;
-    for (int s = 0; s < nsteps; ++s) launch_step(P, U, st, dt_sched + (size_t)s * P->ncases);
+    for (int s = 0; s < nsteps; ++s) launch_step(P, U, st, dt_sched + (size_t)s * P->ncases, s);
     PHX_CK(hipGetLastError());
     return PHX_OK;
 }
@@ -976,8 +1023,9 @@ int phx_run_record(phx_plan* P, double* U, int32_t nsteps, const double* dt_sche
     // step), so only the first input is copied.
     PHX_CK(hipMemcpyAsync(stages, U, len * sizeof(double), hipMemcpyDeviceToDevice, st));
     for (int n = 0; n < nsteps; ++n) {
-        hipLaunchKernelGGL(k_finalize, dim3(1), dim3(FIN_THREADS), 0, st, P->ncases, P->nslot, P->ph.cfl, P->dtmin, P->tfinal, P->t,
-                           P->dt, P->step, P->bad, dt_sched + (size_t)n * P->ncases, 1);
+        const double* frozen = dt_sched + (size_t)n * P->ncases;
+        open_step(P, n, frozen, st);
+        const InStep step{n, frozen};
         double* rec = stages + (size_t)n * S * len;
         double* next = (n + 1 < nsteps) ? rec + (size_t)S * len : U;
         for (int s = 0; s < S; ++s) {
@@ -986,7 +1034,7 @@ int phx_run_record(phx_plan* P, double* U, int32_t nsteps, const double* dt_sche
             M.u_write = next;
             M.s_read = rec + (size_t)s * len;
             M.s_write = (s + 1 < S) ? rec + (size_t)(s + 1) * len : next;  // one-stage tables write S0
-            launch_prog_stage_mapped(P, (size_t)s, M, st);
+            launch_prog_stage_mapped(P, (size_t)s, M, st, &step);
         }
     }
     PHX_CK(hipGetLastError());
@@ -1038,7 +1086,7 @@ int phx_status(phx_plan* P, int32_t* bad_step, int32_t* step, double* t_host, do
     PHX_CK(hipMemcpy(b.data(), P->bad, P->ncases * sizeof(int), hipMemcpyDeviceToHost));
     PHX_CK(hipMemcpy(&s, P->step, sizeof(int), hipMemcpyDeviceToHost));
     if (bad_step)
-        for (int c = 0; c < P->ncases; ++c) bad_step[c] = (b[c] == 0x7fffffff) ? -1 : b[c];
+        for (int c = 0; c < P->ncases; ++c) bad_step[c] = (b[c] == NEVER) ? -1 : b[c];
     if (step) *step = s;
     if (t_host) PHX_CK(hipMemcpy(t_host, P->t, P->ncases * sizeof(double), hipMemcpyDeviceToHost));
     if (dt_host) PHX_CK(hipMemcpy(dt_host, P->dt, P->ncases * sizeof(double), hipMemcpyDeviceToHost));

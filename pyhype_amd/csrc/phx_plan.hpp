@@ -13,6 +13,7 @@
 namespace phx {
 namespace stage {
 struct DevItem;  // a work item with its block's descriptor (phx_stage.hpp)
+struct StepFold; // what closes one step and opens the next (phx_stage.hpp)
 }
 namespace host {
 
@@ -117,9 +118,12 @@ struct phx_plan {
     double* sbuf[2] = {nullptr, nullptr};
     double* acc[phx::host::MAX_ACC] = {};
     double *dt = nullptr, *t = nullptr, *tfinal = nullptr;
-    unsigned long long* dtmin = nullptr;  // nslot partial CFL minima per case, one cache line each
+    // two sets (the step in progress reads one and writes the other) of nslot partial CFL minima per
+    // case, one cache line each
+    unsigned long long* dtmin = nullptr;
     int nslot = 1;
     int *step = nullptr, *bad = nullptr;
+    phx::stage::StepFold* fold = nullptr;  // on the device: where the stage kernels find the above
     long long* dghost_off = nullptr;
     hipStream_t cap_stream = nullptr;
     hipEvent_t ev_a = nullptr, ev_b = nullptr;
@@ -127,9 +131,10 @@ struct phx_plan {
     // (fork/join through ev_fork/ev_join; captured into the step graphs as parallel branches)
     hipStream_t side_stream = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
-    // captured steps: [0] one step, [1] GRAPH_STEPS steps (replayed by phx_run)
-    hipGraphExec_t gexec[2] = {nullptr, nullptr};
-    hipGraph_t graph[2] = {nullptr, nullptr};
+    // captured steps: graph g holds 2^g steps (replayed by phx_run)
+    static constexpr int GRAPHS = 4;
+    hipGraphExec_t gexec[GRAPHS] = {};
+    hipGraph_t graph[GRAPHS] = {};
     double* graph_U = nullptr;
     bool copy_back = false;  // one-stage tables: result lands in sbuf[0] and is copied to U
 

@@ -56,6 +56,30 @@ struct DevItem {
 // Outlined (s_swappc) item functions of the HLLL Gauss-face and generic shared-halo kernels, which
 // appeared when the HLLL norm grew, returned NaN residuals on gfx950 (ROCm 7.2) where the same
 // source inlined, and a stand-alone kernel of the same flux, are bit-exact.
+
+// Closing one step and opening the next: the time steps from the CFL minima of the state (or a given
+// schedule), the times and the step counter.  As a kernel of its own between two steps this took 2.7 to
+// 4.6 us and a launch gap; the stage kernels take it along in extra workgroups instead, where nothing
+// waits for it:
+//  * FOLD_ALL: the first kernel of a step's first stage that only reconstructs, into scratch (split and
+//    element-wise stages); the step's later kernels read dt.
+//  * FOLD_DT, FOLD_TIME: the shared-halo stage needs dt in the step's only kernel per stage, so in the
+//    first stage every update wave takes the minimum itself while extra workgroups store dt and the
+//    counter, and in the second, when nobody reads them any more, the times and the cleared minima.
+// The minima are kept in two sets, read and written by turns, since a two-stage step writes the next
+// step's minima in the launch that clears this step's.
+enum { FOLD_NONE = 0, FOLD_ALL, FOLD_DT, FOLD_TIME };
+constexpr int NEVER = 0x7fffffff;  // bad[] of a case that never failed
+struct StepFold {  // in device memory, read where it is used: as kernel arguments it costs every wave registers
+    int ncases;
+    double cfl;
+    unsigned long long* dtmin;
+    const double* tfinal;
+    double* t;
+    double* dt;
+    int* step;
+};
+
 struct StageArgs {
     const DevBlock* blocks;
     const DevItem* items;
@@ -80,6 +104,11 @@ struct StageArgs {
     double* ff;        // element-wise stage: face fluxes (4 doubles per face, DevBlock::foff)
     int nslot;         // partial CFL minima per case
     int fq;            // flat y-face stage: LDS faces per lane
+    int fold_mode;     // what the launch takes along (FOLD_*), for the minima's set fold_set
+    int fold_set;
+    int fold_blocks;   // extra workgroups of this launch, behind the others
+    const StepFold* fold;
+    const double* frozen;  // the schedule's time steps instead of the CFL minima
     Phys ph;
 };
 
@@ -94,9 +123,51 @@ __device__ __forceinline__ const T& const_ref(const T* p, long i) {
 // Whether the block's case became unrealizable at an earlier step: it is frozen, as the reference aborts
 // that run (Euler2D.py:144-152).  Scalar loads (a lane that fails in this stage writes the current step,
 // which leaves the comparison as it is); a kernel asks after it has issued its first loads, which do
-// not wait for the answer then.
+// not wait for the answer then.  In a launch whose extra workgroups advance the counter the answer does not
+// depend on it where states are written (FOLD_DT: every failure on record is an earlier step's); a
+// FOLD_ALL launch writes scratch only, which the step's next kernel does not use for a frozen case.
 __device__ __forceinline__ bool frozen_case(const StageArgs& A, const DevBlock& B) {
-    return A.skip_dead && ld_const(A.bad, B.case_id) < ld_const(A.step, 0);
+    return A.skip_dead && ld_const(A.bad, B.case_id) < (A.fold_mode == FOLD_DT ? NEVER : ld_const(A.step, 0));
+}
+
+// dt of case c, which an aligned group of nslot lanes asks for together: CFL * minimum, clipped to
+// t_final - t (solvers/base.py:126-136)
+__device__ __forceinline__ double step_dt(const StageArgs& A, int c) {
+    if (A.frozen != nullptr) return A.frozen[c];
+    const StepFold& F = const_ref(A.fold, 0);
+    unsigned long long m = F.dtmin[dt_slot(A.fold_set * F.ncases + c, threadIdx.x & (A.nslot - 1), A.nslot)];
+    const double rem = F.tfinal[c] - F.t[c];
+    for (int o = A.nslot / 2; o > 0; o >>= 1) {
+        const unsigned long long x = __shfl_xor(m, o, A.nslot);
+        m = x < m ? x : m;
+    }
+    const double d = F.cfl * __longlong_as_double((long long)m);
+    return rem < d ? rem : d;
+}
+
+// The extra workgroups of a launch (their first wave; nslot lanes per case); false in the others.
+__device__ __forceinline__ bool fold_step(const StageArgs& A) {
+    const int e = (int)blockIdx.x - ((int)gridDim.x - A.fold_blocks);
+    if (e < 0) return false;
+    const StepFold& F = const_ref(A.fold, 0);
+    if (threadIdx.x >= WAVE) return true;
+    const int c = e * (WAVE / A.nslot) + (int)threadIdx.x / A.nslot;
+    const int g = threadIdx.x & (A.nslot - 1);
+    if (c < F.ncases) {
+        if (A.fold_mode == FOLD_TIME) {
+            if (g == 0) F.t[c] += F.dt[c];
+        } else {
+            double d = step_dt(A, c);
+            if (A.bad[c] != NEVER) d = 0.0;  // a failed case keeps its time
+            if (g == 0) {
+                F.dt[c] = d;
+                if (A.fold_mode == FOLD_ALL) F.t[c] += d;  // Euler2D.py:209
+            }
+        }
+        if (A.fold_mode != FOLD_DT) F.dtmin[dt_slot(A.fold_set * F.ncases + c, g, A.nslot)] = DT_INF_BITS;
+    }
+    if (A.fold_mode != FOLD_TIME && e == 0 && threadIdx.x == 0) F.step[0] += 1;
+    return true;
 }
 
 // cross-lane moves of a 4-vector
@@ -322,8 +393,8 @@ __device__ __forceinline__ void stage_item(const StageArgs& A, const DevItem& it
 // Work distribution: 8 XCDs receive workgroups round-robin; each XCD gets a contiguous range of the
 // (spatially ordered) work list so that halo rows/columns shared by neighbouring items are reused
 // from the same L2.
-__device__ __forceinline__ void item_range(int n, int& lo, int& hi, int& first, int& stride) {
-    const int G = gridDim.x, w = blockIdx.x;
+__device__ __forceinline__ void item_range(int n, int& lo, int& hi, int& first, int& stride, int extra = 0) {
+    const int G = (int)gridDim.x - extra, w = blockIdx.x;
     if (G >= 8) {
         const int x = w & 7;
         lo = (int)(((long)n * x) >> 3);
@@ -502,7 +573,8 @@ __device__ __forceinline__ void stage_wg_item(const StageArgs& A, const DevItem&
     const int k = it.r0 + u;
     Q4 pre[EMIT_CHUNK];
     double LW = 0.0, LE = 0.0, LS = 0.0, LN = 0.0, Ac = 1.0, dxc = 0.0;
-    const double dt = (A.dt != nullptr) ? ld_const(A.dt, B.case_id) : 0.0;
+    const double dt = A.fold_mode == FOLD_DT ? step_dt(A, B.case_id)
+                                             : (A.dt != nullptr ? ld_const(A.dt, B.case_id) : 0.0);
     if (row && owner) {
         cell_L<CART>(B, k, j, LW, LE, LS, LN, Ac);
         prefetch_sources(A, B, k, j, pre);
@@ -528,9 +600,10 @@ __device__ __forceinline__ void stage_wg_item(const StageArgs& A, const DevItem&
 
 template <bool CART, int FLUX, int R, bool GEN>
 __global__ void __launch_bounds__(wg_waves(R) * WAVE) k_stage_wg(StageArgs A) {
+    if (fold_step(A)) return;
     __shared__ double lds[wg_lds(R)];
     int lo, hi, first, stride;
-    item_range(A.nitems, lo, hi, first, stride);
+    item_range(A.nitems, lo, hi, first, stride, A.fold_blocks);
     for (int i = first; i < hi; i += stride) {
         stage_wg_item<CART, FLUX, R, GEN>(A, const_ref(A.items, i), lds);
         __syncthreads();  // the next item reuses the exchange buffers
@@ -1211,8 +1284,9 @@ __global__ void __launch_bounds__(WAVE) k_yface_update(StageArgs A) {
 
 template <int CK, int FLUX, int MINW, bool GEN>
 __global__ void __launch_bounds__(WAVE, MINW) k_recon_x(StageArgs A) {
+    if (fold_step(A)) return;
     int lo, hi, first, stride;
-    item_range(A.nitems, lo, hi, first, stride);
+    item_range(A.nitems, lo, hi, first, stride, A.fold_blocks);
     for (int i = first; i < hi; i += stride) {
         const DevItem& it = const_ref(A.items, i);
         if (CK == 2) {
@@ -1295,8 +1369,9 @@ __device__ __forceinline__ void recon_x_lin_item(const StageArgs& A, const DevIt
 
 template <int CK, int FLUX, int MINW, bool GEN>
 __global__ void __launch_bounds__(WAVE, MINW) k_recon_x_lin(StageArgs A) {
+    if (fold_step(A)) return;
     int lo, hi, first, stride;
-    item_range(A.nitems, lo, hi, first, stride);
+    item_range(A.nitems, lo, hi, first, stride, A.fold_blocks);
     for (int i = first; i < hi; i += stride) {
         const DevItem& it = const_ref(A.items, i);
         if (CK == 2) {
@@ -1319,8 +1394,9 @@ __global__ void __launch_bounds__(WAVE) k_yface(StageArgs A) {
 // not set by the nq-point path
 template <bool CART, int FLUX>
 __global__ void __launch_bounds__(WAVE, 2) k_recon_x_q(StageArgs A) {
+    if (fold_step(A)) return;
     int lo, hi, first, stride;
-    item_range(A.nitems, lo, hi, first, stride);
+    item_range(A.nitems, lo, hi, first, stride, A.fold_blocks);
     for (int i = first; i < hi; i += stride) recon_x_item_q<CART, FLUX>(A, const_ref(A.items, i));
 }
 
@@ -1428,8 +1504,9 @@ __device__ __forceinline__ void ew_update_tile(const StageArgs& A, const DevItem
 
 template <int CK, bool GEN>
 __global__ void __launch_bounds__(EW_WG) k_ew_recon(StageArgs A) {
+    if (fold_step(A)) return;
     int lo, hi, first, stride;
-    item_range(A.nitems, lo, hi, first, stride);
+    item_range(A.nitems, lo, hi, first, stride, A.fold_blocks);
     for (int i = first; i < hi; i += stride) {
         const DevItem& it = const_ref(A.items, i);
         if (CK == 2) {  // items of both geometry kinds: the path of the item's block

@@ -24,7 +24,7 @@ void k_recon_x_lin_tag::launch(const phx_plan* P, int kind, int minw, dim3 g, hi
 void launch_recon_x_lin_mixed(const phx_plan* P, StageArgs A, hipStream_t st) {
     A.items = P->ditems_m[2];
     A.nitems = P->n_m[2];
-    const dim3 g(P->grid_m[2]), b(WAVE);
+    const dim3 g(P->grid_m[2] + A.fold_blocks), b(WAVE);
     const bool gen = generic_instance(P), roe = P->flux == PHX_FLUX_ROE;
     const bool w4 = !gen && P->waves_per_simd >= 4;  // the register budgets the per-kind launches use
 #define PHX_RX(F, M, G) hipLaunchKernelGGL((k_recon_x_lin<2, F, M, G>), g, b, 0, st, A)

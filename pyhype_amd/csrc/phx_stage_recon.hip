@@ -27,7 +27,7 @@ void k_recon_x_tag::launch(const phx_plan* P, int kind, int minw, dim3 g, hipStr
 void launch_recon_x_mixed(const phx_plan* P, StageArgs A, hipStream_t st) {
     A.items = P->ditems_m[0];
     A.nitems = P->n_m[0];
-    const dim3 g(P->grid_m[0]), b(WAVE);
+    const dim3 g(P->grid_m[0] + A.fold_blocks), b(WAVE);
     const bool gen = generic_instance(P), roe = P->flux == PHX_FLUX_ROE;
     const bool w4 = !gen && P->waves_per_simd >= 4;  // the register budgets the per-kind launches use
 #define PHX_RX(F, M, G) hipLaunchKernelGGL((k_recon_x<2, F, M, G>), g, b, 0, st, A)

@@ -58,7 +58,7 @@ void k_ew_update_tag::launch(const phx_plan* P, int kind, int minw, dim3 g, hipS
 void launch_ew_mixed(const phx_plan* P, StageArgs A, int p, hipStream_t st) {
     A.items = P->ditems_em[p];
     A.nitems = P->n_em[p];
-    const dim3 g(P->grid_em[p]), b(EW_WG);
+    const dim3 g(P->grid_em[p] + (p == 0 ? A.fold_blocks : 0)), b(EW_WG);
     const bool gen = generic_instance(P), roe = P->flux == PHX_FLUX_ROE;
     if (p == 0) {
         if (gen) hipLaunchKernelGGL((k_ew_recon<2, true>), g, b, 0, st, A);
