@@ -412,8 +412,8 @@ int build_items(phx_plan* P) {
         rc = upload_items(P, P->items_e[p], P->ditems_e[p], P->grid_e[p], P->grid_waves);
         if (rc) return rc;
     }
-    // both geometry kinds: one list per phase of the element-wise stage and of the split stages 6
-    // and 7 with midpoint faces (one launch instead of two; the kernels choose the path per block)
+    // both geometry kinds: one list of the shared-halo stage, and per phase of the element-wise stage and of
+    // the split stages 6 and 7 with midpoint faces (one launch instead of two; the kernels choose the path per block)
     auto merge = [&](const std::vector<WorkItem> (&two)[2], DevItem*& dev, int& n_out, int& grid_out) -> int {
         if (two[0].empty() || two[1].empty()) return PHX_OK;
         std::vector<WorkItem> both(two[0]);
@@ -431,6 +431,10 @@ int build_items(phx_plan* P) {
             rc = merge(P->items_e[p], P->ditems_em[p], P->n_em[p], P->grid_em[p]);
             if (rc) return rc;
         }
+    if (P->variant == 2) {
+        rc = merge(P->items, P->ditems_m[0], P->n_m[0], P->grid_m[0]);
+        if (rc) return rc;
+    }
     if ((P->variant == 6 || P->variant == 7) && P->ph.nq == 1) {
         rc = merge(P->items_b, P->ditems_m[1], P->n_m[1], P->grid_m[1]);
         if (rc) return rc;
@@ -642,6 +646,10 @@ void launch_stage(phx_plan* P, StageArgs A, hipStream_t st) {
     }
     if (P->variant == 2) {
         A.rows_wave = wg_rows(P->rows_per_item);
+        if (P->ditems_m[0]) {
+            launch_stage_wg_mixed(P, A, st);
+            return;
+        }
         for_kinds(P, !P->items[0].empty(), !P->items[1].empty(), st, [&](int kind, hipStream_t s) {
             launch_kind<k_stage_wg_tag>(P, A, kind, P->ditems[kind], (int)P->items[kind].size(), P->grid[kind],
                                         2, s);

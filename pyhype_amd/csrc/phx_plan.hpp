@@ -99,7 +99,7 @@ struct phx_plan {
     // list (one launch; the kernels pick the geometry path per block)
     phx::stage::DevItem* ditems_em[3] = {};
     int n_em[3] = {0, 0, 0}, grid_em[3] = {0, 0, 0};
-    // split stages 6 and 7 likewise: merged lists of items (variant 6 reconstruction), items_b (y-faces
+    // shared-halo stage and split stages 6 and 7 likewise: merged lists of items (variant 2, variant 6 reconstruction), items_b (y-faces
     // and update) and items_f (variant 7 reconstruction)
     phx::stage::DevItem* ditems_m[3] = {};
     int n_m[3] = {0, 0, 0}, grid_m[3] = {0, 0, 0};

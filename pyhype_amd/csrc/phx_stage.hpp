@@ -598,14 +598,21 @@ __device__ __forceinline__ void stage_wg_item(const StageArgs& A, const DevItem&
     reduce_item(A, B, lane, lane_dt, lane_bad);
 }
 
-template <bool CART, int FLUX, int R, bool GEN>
+// CK: geometry kind of the launch's blocks, 0 general, 1 Cartesian, 2 both
+template <int CK, int FLUX, int R, bool GEN>
 __global__ void __launch_bounds__(wg_waves(R) * WAVE) k_stage_wg(StageArgs A) {
     if (fold_step(A)) return;
     __shared__ double lds[wg_lds(R)];
     int lo, hi, first, stride;
     item_range(A.nitems, lo, hi, first, stride, A.fold_blocks);
     for (int i = first; i < hi; i += stride) {
-        stage_wg_item<CART, FLUX, R, GEN>(A, const_ref(A.items, i), lds);
+        const DevItem& it = const_ref(A.items, i);
+        if (CK == 2) {
+            if (it.b.kind == PHX_GEOM_CARTESIAN) stage_wg_item<true, FLUX, R, GEN>(A, it, lds);
+            else stage_wg_item<false, FLUX, R, GEN>(A, it, lds);
+        } else {
+            stage_wg_item<CK == 1, FLUX, R, GEN>(A, it, lds);
+        }
         __syncthreads();  // the next item reuses the exchange buffers
     }
 }
@@ -1155,17 +1162,6 @@ __device__ __forceinline__ void yface_update_wg_item(const StageArgs& A, const D
     const int j = it.j0 + lane;
     const int nrow = it.r1 - it.r0;
     const Phys ph = A.ph;
-#ifdef YPRE
-    // the cell's own values with the face states: they arrive while the flux is computed
-    const bool own = w < nrow && j < nx;
-    Q4 p, pre[EMIT_CHUNK];
-    double LW, LE, LS, LN, Ac;
-    if (own) {
-        p = ld4(A.p1 + B.off + 4 * ((long)(it.r0 + w) * nx + j));
-        cell_L<CART>(B, it.r0 + w, j, LW, LE, LS, LN, Ac);
-        if (YPRE > 1) prefetch_sources(A, B, it.r0 + w, j, pre);
-    }
-#endif
     const bool dead = frozen_case(A, B);
     if (dead) return;  // uniform over the workgroup
     if (w <= nrow && j < nx) {
@@ -1179,11 +1175,9 @@ __device__ __forceinline__ void yface_update_wg_item(const StageArgs& A, const D
         const int k = it.r0 + w;
         const double dt = (A.dt != nullptr) ? ld_const(A.dt, B.case_id) : 0.0;
         const Q4 FS = lds[w * WAVE + lane], FN = lds[(w + 1) * WAVE + lane];
-#ifndef YPRE
         const Q4 p = ld4(A.p1 + B.off + 4 * ((long)k * nx + j));
         double LW, LE, LS, LN, Ac;
         cell_L<CART>(B, k, j, LW, LE, LS, LN, Ac);
-#endif
         Q4 Res;
         if (Q) {  // the face entries are the Gauss sums already
 #pragma unroll
@@ -1609,6 +1603,7 @@ struct k_update_tag {
 // of phase p (0 reconstruction, 1 faces, 2 update) of the element-wise stage, of the reconstruction of
 // variants 6 and 7, and of the y-face and update kernel of variants 6 and 7.
 void launch_ew_mixed(const phx_plan* P, StageArgs A, int p, hipStream_t st);
+void launch_stage_wg_mixed(const phx_plan* P, StageArgs A, hipStream_t st);
 void launch_recon_x_mixed(const phx_plan* P, StageArgs A, hipStream_t st);
 void launch_recon_x_lin_mixed(const phx_plan* P, StageArgs A, hipStream_t st);
 void launch_yface_wg_mixed(const phx_plan* P, StageArgs A, hipStream_t st);

@@ -8,8 +8,9 @@ namespace {
 struct k_stage_wg_go {
     template <bool C, int F, int M, bool G>
     static void go(dim3 g, hipStream_t st, const StageArgs& A) {
-        if (A.rows_wave == 1) hipLaunchKernelGGL((k_stage_wg<C, F, 1, G>), g, dim3(wg_waves(1) * WAVE), 0, st, A);
-        else hipLaunchKernelGGL((k_stage_wg<C, F, 2, G>), g, dim3(wg_waves(2) * WAVE), 0, st, A);
+        constexpr int K = C ? 1 : 0;
+        if (A.rows_wave == 1) hipLaunchKernelGGL((k_stage_wg<K, F, 1, G>), g, dim3(wg_waves(1) * WAVE), 0, st, A);
+        else hipLaunchKernelGGL((k_stage_wg<K, F, 2, G>), g, dim3(wg_waves(2) * WAVE), 0, st, A);
     }
 };
 struct k_stage_pair_go {
@@ -41,6 +42,20 @@ struct k_ew_update_go {
 
 void k_stage_wg_tag::launch(const phx_plan* P, int kind, int minw, dim3 g, hipStream_t st, const StageArgs& A) {
     dispatch<k_stage_wg_go>(P, kind, minw, g, st, A);
+}
+// one launch over the merged list of both geometry kinds
+template <int F, bool G>
+static void launch_wg_both(dim3 g, hipStream_t st, const StageArgs& A) {
+    if (A.rows_wave == 1) hipLaunchKernelGGL((k_stage_wg<2, F, 1, G>), g, dim3(wg_waves(1) * WAVE), 0, st, A);
+    else hipLaunchKernelGGL((k_stage_wg<2, F, 2, G>), g, dim3(wg_waves(2) * WAVE), 0, st, A);
+}
+void launch_stage_wg_mixed(const phx_plan* P, StageArgs A, hipStream_t st) {
+    A.items = P->ditems_m[0];
+    A.nitems = P->n_m[0];
+    const dim3 g(P->grid_m[0] + A.fold_blocks);
+    const bool gen = generic_instance(P);
+    if (P->flux == PHX_FLUX_ROE) gen ? launch_wg_both<0, true>(g, st, A) : launch_wg_both<0, false>(g, st, A);
+    else gen ? launch_wg_both<1, true>(g, st, A) : launch_wg_both<1, false>(g, st, A);
 }
 void k_stage_pair_tag::launch(const phx_plan* P, int kind, int minw, dim3 g, hipStream_t st, const StageArgs& A) {
     dispatch<k_stage_pair_go>(P, kind, minw, g, st, A);

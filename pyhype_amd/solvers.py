@@ -85,8 +85,8 @@ def validate_config(config) -> List[List[float]]:
 #    of the chip: with one row each up to 256 workgroups (64^2: 11.0 against 14.6 with the split
 #    stage and 25.7 fused; 8 x 32^2: 11.1 against 15.9), with two rows up to 384 (128^2, 192 of them:
 #    11.7 against 14.9; six 93 x 61 HLLL blocks, 372: 25.5 against 32.4).  At 500 it falls behind (5 x
-#    100^2 HLLL: 26.3 against 22.5).  A mesh of both geometry kinds takes two launches of it, the
-#    split stage one per kernel over both (4 x 50^2: 29.2 against 22.5).
+#    100^2 HLLL: 26.3 against 22.5; 4 x 70^2 of both geometry kinds, 560 and 280: 26.8 and 21.8 against
+#    21.0).
 #  * The split stage with one y-face per wave up to the size where the states that pass between its
 #    kernels no longer stay in the caches: strips (variant 6) while a Cartesian mesh has fewer than 10^5
 #    cells (256^2: 18.2 against 20.4), row-major (variant 7) beyond (400^2: 26.6 against 27.4;
@@ -117,7 +117,7 @@ def default_shape(plan) -> dict:
     kinds = {e.cartesian for e in plan.blocks}
     strips = [(-(-e.nx // 60), e.ny) for e in plan.blocks]
     for rows, most in zip((1, 2), SHARED_ITEMS):
-        if len(kinds) == 1 and sum(n * -(-ny // rows) for n, ny in strips) <= most:
+        if sum(n * -(-ny // rows) for n, ny in strips) <= most:
             return {"rows_per_item": rows, "variant": 2}
     if cells > SPLIT_CELLS[plan.flux]:
         return {"rows_per_item": max(FUSED_ROWS, default_rows(cells))}

@@ -16,7 +16,8 @@ def plan(sizes, cartesian=True, flux="Roe", nq=1):
 @pytest.mark.parametrize("p, variant, rows", [
     (plan([(1, 1)]), 2, 1), (plan([(60, 256)]), 2, 1), (plan([(61, 128)]), 2, 1), (plan([(60, 257)]), 2, 2),
     (plan([(61, 129)]), 2, 2), (plan([(60, 768)]), 2, 2), (plan([(60, 769)]), 6, 1),
-    (plan([(50, 50)] * 4, (True, False, False, False), "HLLL"), 6, 1),
+    (plan([(50, 50)] * 4, (True, False, False, False), "HLLL"), 2, 1),
+    (plan([(80, 100)] * 4, (True, False, False, False), "HLLL"), 6, 1),
     (plan([(60, 769)], False), 7, 1), (plan([(400, 400)]), 7, 1),
     (plan([(1000, 1000)]), 7, 1), (plan([(1000, 1001)]), 0, 8), (plan([(1000, 1001)], True, "HLLL"), 7, 1),
     (plan([(1600, 1600)], False, "HLLL"), 0, 10), (plan([(4000, 4000)]), 0, 64),
