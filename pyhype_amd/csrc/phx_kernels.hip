@@ -392,9 +392,12 @@ int build_items(phx_plan* P) {
         }
     }
     // fused kernel, one workgroup per item: item pairs dealt to the XCDs, half a round of
-    // workgroups per XCD (3 waves on each of its SIMDs) ending on half-size items
+    // workgroups per XCD (3 waves on each of its SIMDs) ending on half-size items, but no more than a sixth
+    // of the items, whose halo rows cost more than the even end gives (1.4 x 10^6 cells, 2,400 items: us
+    // per stage 116 with 192 per XCD, 114 with 48; batch of 2.4 x 10^6, 196 and 192; 64 cases of 6 x 10^6
+    // and 9,800 items the other way, 447 and 464)
     if (P->variant == 0 && P->grid_waves == 0)
-        for (int kind = 0; kind < 2; ++kind) order_for_xcds(P->items[kind], P->ncu * 4 * 3 / 8 / 2);
+        for (int kind = 0; kind < 2; ++kind) order_for_xcds(P->items[kind], std::min(P->ncu * 4 * 3 / 8 / 2, (int)P->items[kind].size() / 8 / 6));
     if (P->variant != 0 && P->grid_waves == 0 && P->xcd_chunk > 0)
         for (int kind = 0; kind < 2; ++kind) {
             deal_to_xcds(P->items[kind], P->xcd_chunk);
