@@ -291,22 +291,28 @@ class DevicePlan:
                                       dt.ctypes.data_as(C.POINTER(C.c_double))), "phx_status")
         return np.array(bad[:], dtype=np.int64), step.value, t, dt
 
-    def failed_cases(self):
-        bad = self.status()[0]
+    def failed_cases(self, bad=None):
+        bad = self.status()[0] if bad is None else bad
         return {c: int(b) for c, b in enumerate(bad) if b >= 0}
 
-    def check_realizable(self):
-        failed = self.failed_cases()
+    def check_realizable(self, bad=None):
+        """Raise if any case failed (``bad``: the failing steps of a ``status()`` at hand)."""
+        failed = self.failed_cases(bad)
         if failed:
             c, b = min(failed.items(), key=lambda kv: kv[1])
             raise RealizabilityError(
                 f"ConservativeState has unrealizable values (rho <= 0 or E <= 0) in case {c} after step {b}"
                 + (f"; failed cases: {failed}" if len(failed) > 1 else ""))
 
+    def _result_like(self, U):
+        """Room for a result in the state layout, every element of which the kernels write."""
+        if U.numel() == self.state_len and U.dtype == self.torch.float64:
+            return self.torch.empty_like(U)
+        return self.torch.zeros_like(U)   # an oversized buffer: the rest stays zero
+
     def residual(self, U=None):
-        torch = self.torch
         U = self.U if U is None else U
-        R = torch.zeros_like(U)
+        R = self._result_like(U)
         nat.check(self.lib.phx_residual(self.handle, self.ptr(U), self.ptr(R), self.stream()), "phx_residual")
         return R
 
@@ -336,14 +342,14 @@ class DevicePlan:
 
     def residual_vjp(self, U, lamR):
         """(dR/dU)^T lamR at state U (device tensors of the state layout)."""
-        lamU = self.torch.zeros_like(U)
+        lamU = self._result_like(U)
         nat.check(self.lib.phx_residual_vjp(self.handle, self.ptr(U), self.ptr(lamR), self.ptr(lamU), self.stream()),
                   "phx_residual_vjp")
         return lamU
 
     def residual_jvp(self, U, dU):
         """(dR/dU) dU at state U (device tensors of the state layout)."""
-        dR = self.torch.zeros_like(U)
+        dR = self._result_like(U)
         nat.check(self.lib.phx_residual_jvp(self.handle, self.ptr(U), self.ptr(dU), self.ptr(dR), self.stream()),
                   "phx_residual_jvp")
         return dR

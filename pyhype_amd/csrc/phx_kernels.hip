@@ -113,15 +113,22 @@ __global__ void __launch_bounds__(FIN_THREADS) k_finalize(int ncases, int nslot,
     __syncthreads();
     if (advance && threadIdx.x == 0) step[0] = s_next;
 }
-__global__ void k_reset(int ncases, int nslot, const double* t0, double* t, unsigned long long* dtmin, int* bad,
+// start times of cases [c0, c0 + RESET_CASES), by value: no buffer, copy or wait for one
+constexpr int RESET_CASES = 64;
+struct StartTimes {
+    double t[RESET_CASES];
+};
+__global__ void k_reset(int ncases, int nslot, int c0, StartTimes T, double* t, unsigned long long* dtmin, int* bad,
                         int* step, int step0) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;  // one thread per (set, case, slot)
-    if (c < 2 * ncases * nslot) dtmin[(long)c * DT_STRIDE] = DT_INF_BITS;
-    if (c < ncases) {
-        t[c] = t0[c];
-        bad[c] = NEVER;
+    if (c0 == 0) {
+        if (c < 2 * ncases * nslot) dtmin[(long)c * DT_STRIDE] = DT_INF_BITS;
+        if (c == 0) step[0] = step0;
     }
-    if (c == 0) step[0] = step0;
+    if (c < RESET_CASES && c0 + c < ncases) {
+        t[c0 + c] = T.t[c];
+        bad[c0 + c] = NEVER;
+    }
 }
 
 __global__ void k_fill_inf(int ncases, int nslot, unsigned long long* dtmin) {
@@ -681,6 +688,16 @@ void launch_dt_reduce(phx_plan* P, const double* U, hipStream_t st) {
     }
 }
 
+void launch_reset(phx_plan* P, const double* t0, int step0, hipStream_t st) {
+    for (int c0 = 0; c0 < P->ncases; c0 += RESET_CASES) {
+        StartTimes T{};
+        std::copy(t0 + c0, t0 + std::min(c0 + RESET_CASES, P->ncases), T.t);
+        const int n = c0 == 0 ? std::max(2 * P->ncases * P->nslot, RESET_CASES) : RESET_CASES;
+        hipLaunchKernelGGL(k_reset, dim3((n + 255) / 256), dim3(256), 0, st, P->ncases, P->nslot, c0, T, P->t, P->dtmin,
+                           P->bad, P->step, step0);
+    }
+}
+
 // Buffers of one stage-program launch: the caller's state U (read as U0 / stage-0 input, written by
 // the last stage) and the stage-state buffer the stage reads (s_read) or writes (s_write).
 struct BufMap {
@@ -789,7 +806,7 @@ int phx_plan_destroy(phx_plan* P) {
                     P->ditems_e[1][0], P->ditems_e[1][1], P->ditems_e[2][0], P->ditems_e[2][1],
                     P->ditems_em[0], P->ditems_em[1], P->ditems_em[2], P->ditems_m[0], P->ditems_m[1],
                     P->ditems_m[2],
-                    P->sbuf[0], P->sbuf[1], P->dt, P->t, P->tfinal, P->dtmin, P->step, P->bad, P->fold, P->dghost_off};
+                    P->sbuf[0], P->sbuf[1], P->t, P->tfinal, P->dtmin, P->fold, P->dghost_off};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (int m = 0; m < MAX_ACC; ++m)
@@ -930,27 +947,21 @@ int phx_plan_create(const phx_plan_desc* D, phx_plan** out) {
     if (D->nstages > 2) PHX_CKP(hipMalloc(&P->sbuf[1], sbytes));
     for (int m = 0; m < P->nacc; ++m) PHX_CKP(hipMalloc(&P->acc[m], sbytes));
     const size_t cb = (size_t)D->ncases * sizeof(double);
-    PHX_CKP(hipMalloc(&P->dt, cb));
-    PHX_CKP(hipMalloc(&P->t, cb));
+    // t, dt, bad and step in one piece, which phx_status copies at once
+    PHX_CKP(hipMalloc(&P->t, 2 * cb + (D->ncases + 1) * sizeof(int)));
+    P->dt = P->t + D->ncases;
+    P->bad = reinterpret_cast<int*>(P->dt + D->ncases);
+    P->step = P->bad + D->ncases;
     PHX_CKP(hipMalloc(&P->tfinal, cb));
     PHX_CKP(hipMalloc(&P->dtmin, (size_t)2 * D->ncases * P->nslot * DT_STRIDE * sizeof(unsigned long long)));
-    PHX_CKP(hipMalloc(&P->step, sizeof(int)));
-    PHX_CKP(hipMalloc(&P->bad, D->ncases * sizeof(int)));
     const StepFold fold{P->ncases, P->ph.cfl, P->dtmin, P->tfinal, P->t, P->dt, P->step};
     PHX_CKP(hipMalloc(&P->fold, sizeof(fold)));
     PHX_CKP(hipMemcpy(P->fold, &fold, sizeof(fold), hipMemcpyHostToDevice));
     PHX_CKP(hipMemcpy(P->tfinal, D->t_final, cb, hipMemcpyHostToDevice));
     PHX_CKP(hipMemset(P->dt, 0, cb));
-    std::vector<double> zeros(D->ncases, 0.0);
-    double* t0 = nullptr;
-    PHX_CKP(hipMalloc(&t0, cb));
-    PHX_CKP(hipMemcpy(t0, zeros.data(), cb, hipMemcpyHostToDevice));
-    hipLaunchKernelGGL(k_reset, dim3((2 * D->ncases * P->nslot + 255) / 256), dim3(256), 0, 0, D->ncases, P->nslot, t0, P->t,
-                       P->dtmin,
-                       P->bad, P->step, 0);
+    launch_reset(P, std::vector<double>(D->ncases, 0.0).data(), 0, nullptr);
     PHX_CKP(hipGetLastError());
     PHX_CKP(hipDeviceSynchronize());
-    PHX_CKP(hipFree(t0));
     rc = phx::host::adjoint_prepare(P);
     if (rc) return bail(rc);
     PHX_CKP(hipStreamCreateWithFlags(&P->cap_stream, hipStreamNonBlocking));
@@ -967,16 +978,9 @@ int phx_plan_create(const phx_plan_desc* D, phx_plan** out) {
 int phx_reset(phx_plan* P, const double* t0_host, int32_t step0, void* stream) {
     if (!P || !t0_host) return fail(PHX_E_INVALID, "null argument");
     hipStream_t st = (hipStream_t)stream;
-    const size_t cb = (size_t)P->ncases * sizeof(double);
-    double* t0 = nullptr;
-    PHX_CK(hipMalloc(&t0, cb));
-    PHX_CK(hipMemcpy(t0, t0_host, cb, hipMemcpyHostToDevice));
-    hipLaunchKernelGGL(k_reset, dim3((2 * P->ncases * P->nslot + 255) / 256), dim3(256), 0, st, P->ncases, P->nslot, t0,
-                       P->t, P->dtmin,
-                       P->bad, P->step, step0);
+    launch_reset(P, t0_host, step0, st);
     PHX_CK(hipGetLastError());
     PHX_CK(hipStreamSynchronize(st));
-    PHX_CK(hipFree(t0));
     return PHX_OK;
 }
 
@@ -1092,15 +1096,16 @@ int phx_ghosts(phx_plan* P, const double* U, double* G, void* stream) {
 int phx_status(phx_plan* P, int32_t* bad_step, int32_t* step, double* t_host, double* dt_host) {
     if (!P) return fail(PHX_E_INVALID, "null argument");
     PHX_CK(hipDeviceSynchronize());
-    std::vector<int> b(P->ncases);
-    int s = 0;
-    PHX_CK(hipMemcpy(b.data(), P->bad, P->ncases * sizeof(int), hipMemcpyDeviceToHost));
-    PHX_CK(hipMemcpy(&s, P->step, sizeof(int), hipMemcpyDeviceToHost));
+    const size_t n = (size_t)P->ncases;
+    std::vector<char> all(2 * n * sizeof(double) + (n + 1) * sizeof(int));
+    PHX_CK(hipMemcpy(all.data(), P->t, all.size(), hipMemcpyDeviceToHost));
+    const double* t = reinterpret_cast<const double*>(all.data());
+    const int* b = reinterpret_cast<const int*>(t + 2 * n);
     if (bad_step)
-        for (int c = 0; c < P->ncases; ++c) bad_step[c] = (b[c] == NEVER) ? -1 : b[c];
-    if (step) *step = s;
-    if (t_host) PHX_CK(hipMemcpy(t_host, P->t, P->ncases * sizeof(double), hipMemcpyDeviceToHost));
-    if (dt_host) PHX_CK(hipMemcpy(dt_host, P->dt, P->ncases * sizeof(double), hipMemcpyDeviceToHost));
+        for (size_t c = 0; c < n; ++c) bad_step[c] = (b[c] == NEVER) ? -1 : b[c];
+    if (step) *step = b[n];
+    if (t_host) std::copy(t, t + n, t_host);
+    if (dt_host) std::copy(t + n, t + 2 * n, dt_host);
     return PHX_OK;
 }
 

@@ -228,7 +228,7 @@ class Euler2DBatch:
         if n <= 0:
             return
         try:
-            self.plan.run(n, use_graph=use_graph, check=self.strict)
+            self.plan.run(n, use_graph=use_graph, check=False)
         finally:
             # also after a RealizabilityError: time, step counter and the failing step of each case
             # describe the state the plan holds
@@ -236,7 +236,9 @@ class Euler2DBatch:
             self.t = t
             self.dt_last = dt
             self.num_time_step = step
-            self.failed = {c: int(b) for c, b in enumerate(bad) if b >= 0}
+            self.failed = self.plan.failed_cases(bad)
+        if self.strict:
+            self.plan.check_realizable(bad)
 
     def autotune(self, steps: int = 10, **kw):
         """Tune the launch shape on the current state (state, time and step are restored)."""
