@@ -29,13 +29,33 @@ using phx::Q4;
 using phx::dev::DevBlock;
 using phx::dev::ld_const;
 using phx::host::AdjBlock;
+using phx::host::AdjItem;
 using phx::host::AdjTile;
 using phx::host::fail;
+
+// A tile with its block's descriptor and offsets: one scalar load before a lane's first address, not two
+// in a row.  These kernels wait for memory half of their time and more (one to four waves per SIMD, each
+// with one round of loads and one of stores); this took 2 % of a 256 x 256 gradient.
+struct phx::host::AdjItem {
+    int block, start, count;
+    DevBlock b;
+    AdjBlock o;
+};
 
 namespace {
 
 constexpr int TILE = 256;
+
+// Position of this workgroup in the launch's tiles: each of the 8 XCDs, which take workgroups in turn, gets
+// a contiguous range, so that a row's stencil finds its neighbour rows in the same L2 (256 x 256 cells:
+// k_adj_gather 6.9 -> 5.3 us, k_adj_face 15.0 -> 14.0; the value and the gradient over 20 SSPRK2 steps 2,943 ->
+// 2,829).
+__device__ __forceinline__ int tile_pos() {
+    const int n = (int)gridDim.x, x = (int)blockIdx.x & 7, q = n >> 3, r = n & 7;
+    return x * q + (x < r ? x : r) + ((int)blockIdx.x >> 3);
+}
 constexpr int MAX_TERMS = PHX_MAX_STAGES + 2;
+constexpr int FIRST_TERMS = 3;
 
 // sum_m c_m * (dt of the cell's case if scaled_m) * in_m at one cell: the residual seeds and the
 // output terms of a Runge-Kutta step VJP, evaluated where they are used
@@ -48,15 +68,19 @@ struct Terms {
 };
 
 __device__ __forceinline__ Q4 eval_terms(const Terms& T, const DevBlock& B, long long cell) {
-    Q4 r = phx::q4zero();
+    Q4 r = phx::q4zero(), x[FIRST_TERMS];
     const double dt = T.dt ? T.dt[B.case_id] : 1.0;
+    // the first terms are loaded together: a two-stage step has no more
+#pragma unroll
+    for (int m = 0; m < FIRST_TERMS; ++m)
+        if (m < T.n) x[m] = phx::adj::ld(T.in[m] + 4 * cell);
 #pragma unroll
     for (int m = 0; m < MAX_TERMS; ++m) {
         if (m >= T.n) break;
         const double c = T.scaled[m] ? T.c[m] * dt : T.c[m];
-        const double* p = T.in[m] + 4 * cell;
+        const Q4 y = m < FIRST_TERMS ? x[m < FIRST_TERMS ? m : 0] : phx::adj::ld(T.in[m] + 4 * cell);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) r.v[q] += c * p[q];
+        for (int q = 0; q < 4; ++q) r.v[q] += c * y.v[q];
     }
     return r;
 }
@@ -69,13 +93,13 @@ struct TermSeed {
 // NQ: 1 (midpoint faces) or phx::QMAX (nq = ph.nq Gauss points per face); the point records are
 // RB*nq doubles per cell and FA*nq per face
 template <int FLUX, int NQ>
-__global__ void __launch_bounds__(TILE) k_adj_face(const DevBlock* blocks, const AdjBlock* offs, const AdjTile* tiles,
+__global__ void __launch_bounds__(TILE) k_adj_face(const DevBlock* blocks, const AdjBlock* offs, const AdjItem* tiles,
                                                    const double* U, const double* rb, Terms kappa, double* fadj,
                                                    Phys ph) {
-    const AdjTile t = ld_const(tiles, blockIdx.x);
+    const AdjItem t = ld_const(tiles, tile_pos());
     if ((int)threadIdx.x >= t.count) return;
-    const DevBlock B = ld_const(blocks, t.block);  // descriptor in scalar registers
-    const AdjBlock O = ld_const(offs, t.block);
+    const DevBlock& B = t.b;  // in scalar registers
+    const AdjBlock& O = t.o;
     const long long f = (long long)t.start + threadIdx.x;
     double* out = fadj + (long long)phx::adj::FA * phx::adj::npts<NQ>(ph) * (O.face + f);
     const TermSeed seed{kappa};
@@ -84,12 +108,12 @@ __global__ void __launch_bounds__(TILE) k_adj_face(const DevBlock* blocks, const
 }
 
 template <int NQ>
-__global__ void __launch_bounds__(TILE) k_adj_recon(const DevBlock* blocks, const AdjBlock* offs, const AdjTile* tiles,
+__global__ void __launch_bounds__(TILE) k_adj_recon(const DevBlock* blocks, const AdjBlock* offs, const AdjItem* tiles,
                                                     const double* U, double* rb, Phys ph) {
-    const AdjTile t = ld_const(tiles, blockIdx.x);
+    const AdjItem t = ld_const(tiles, tile_pos());
     if ((int)threadIdx.x >= t.count) return;
-    const DevBlock B = ld_const(blocks, t.block);  // descriptor in scalar registers
-    const AdjBlock O = ld_const(offs, t.block);
+    const DevBlock& B = t.b;  // in scalar registers
+    const AdjBlock& O = t.o;
     const int e = t.start + threadIdx.x;
     const int k = e / B.nx, j = e - k * B.nx;
     double* out = rb + (long long)phx::adj::RB * phx::adj::npts<NQ>(ph) * phx::adj::cell_index(O, B, k, j);
@@ -98,12 +122,12 @@ __global__ void __launch_bounds__(TILE) k_adj_recon(const DevBlock* blocks, cons
 }
 
 template <int NQ>
-__global__ void __launch_bounds__(TILE) k_adj_cell(const DevBlock* blocks, const AdjBlock* offs, const AdjTile* tiles,
+__global__ void __launch_bounds__(TILE) k_adj_cell(const DevBlock* blocks, const AdjBlock* offs, const AdjItem* tiles,
                                                    const double* U, const double* fadj, double* slot, Phys ph) {
-    const AdjTile t = ld_const(tiles, blockIdx.x);
+    const AdjItem t = ld_const(tiles, tile_pos());
     if ((int)threadIdx.x >= t.count) return;
-    const DevBlock B = ld_const(blocks, t.block);  // descriptor in scalar registers
-    const AdjBlock O = ld_const(offs, t.block);
+    const DevBlock& B = t.b;  // in scalar registers
+    const AdjBlock& O = t.o;
     const int e = t.start + threadIdx.x;
     const int k = e / B.nx, j = e - k * B.nx;
     double* out = slot + phx::adj::SLOT * phx::adj::cell_index(O, B, k, j);
@@ -111,18 +135,27 @@ __global__ void __launch_bounds__(TILE) k_adj_cell(const DevBlock* blocks, const
     else phx::adj::cell_adj<false, NQ>(blocks, B, U, O, fadj, k, j, out, ph);
 }
 
-// Midpoint faces: the reconstruction and its VJP with one lane per cell and variable (4*TILE lanes
-// per tile of TILE cells): four times the waves of the per-cell kernels on the same tiles, and the
-// registers of one variable's chain.
-constexpr int VTILE = 4 * TILE;
+// Midpoint faces: the reconstruction and its VJP with one lane per cell and variable: four times the
+// waves of the per-cell kernels, and the registers of one variable's chain.  Four workgroups of TILE lanes
+// to a tile of TILE cells: as one of 4*TILE lanes a small mesh kept a quarter of the CUs busy (160 x 96
+// cells, k_tan_recon_v: 13.0 us, 9.8 now; one lane per cell, k_tan_recon, 16.1).
+constexpr int VPARTS = 4;
+constexpr int VCELLS = TILE / VPARTS;
+// the tile of this workgroup and its cell of it
+__device__ __forceinline__ AdjItem part_tile(const AdjItem* tiles, int& c, int& v) {
+    const int w = tile_pos();
+    c = (w % VPARTS) * VCELLS + ((int)threadIdx.x >> 2);
+    v = (int)threadIdx.x & 3;
+    return ld_const(tiles, w / VPARTS);
+}
 
-__global__ void __launch_bounds__(VTILE) k_adj_recon_v(const DevBlock* blocks, const AdjBlock* offs,
-                                                       const AdjTile* tiles, const double* U, double* rb, Phys ph) {
-    const AdjTile t = ld_const(tiles, blockIdx.x);
-    const int c = (int)threadIdx.x >> 2, v = (int)threadIdx.x & 3;
+__global__ void __launch_bounds__(TILE) k_adj_recon_v(const DevBlock* blocks, const AdjBlock* offs,
+                                                       const AdjItem* tiles, const double* U, double* rb, Phys ph) {
+    int c, v;
+    const AdjItem t = part_tile(tiles, c, v);
     if (c >= t.count) return;
-    const DevBlock B = ld_const(blocks, t.block);  // descriptor in scalar registers
-    const AdjBlock O = ld_const(offs, t.block);
+    const DevBlock& B = t.b;  // in scalar registers
+    const AdjBlock& O = t.o;
     const int e = t.start + c;
     const int k = e / B.nx, j = e - k * B.nx;
     double* out = rb + (long long)phx::adj::RB * phx::adj::cell_index(O, B, k, j);
@@ -130,14 +163,14 @@ __global__ void __launch_bounds__(VTILE) k_adj_recon_v(const DevBlock* blocks, c
     else phx::adj::recon_cell_var<false>(blocks, B, U, k, j, v, out, ph);
 }
 
-__global__ void __launch_bounds__(VTILE) k_adj_cell_v(const DevBlock* blocks, const AdjBlock* offs,
-                                                      const AdjTile* tiles, const double* U, const double* fadj,
+__global__ void __launch_bounds__(TILE) k_adj_cell_v(const DevBlock* blocks, const AdjBlock* offs,
+                                                      const AdjItem* tiles, const double* U, const double* fadj,
                                                       double* slot, Phys ph) {
-    const AdjTile t = ld_const(tiles, blockIdx.x);
-    const int c = (int)threadIdx.x >> 2, v = (int)threadIdx.x & 3;
+    int c, v;
+    const AdjItem t = part_tile(tiles, c, v);
     if (c >= t.count) return;
-    const DevBlock B = ld_const(blocks, t.block);  // descriptor in scalar registers
-    const AdjBlock O = ld_const(offs, t.block);
+    const DevBlock& B = t.b;  // in scalar registers
+    const AdjBlock& O = t.o;
     const int e = t.start + c;
     const int k = e / B.nx, j = e - k * B.nx;
     double* out = slot + phx::adj::SLOT * phx::adj::cell_index(O, B, k, j);
@@ -147,32 +180,34 @@ __global__ void __launch_bounds__(VTILE) k_adj_cell_v(const DevBlock* blocks, co
 
 // lamU = (dR/dU)^T kappa + extra terms (pointwise; extra may include lamU itself)
 template <int NQ>
-__global__ void __launch_bounds__(TILE) k_adj_gather(const DevBlock* blocks, const AdjBlock* offs, const AdjTile* tiles,
+__global__ void __launch_bounds__(TILE) k_adj_gather(const DevBlock* blocks, const AdjBlock* offs, const AdjItem* tiles,
                                                      const double* slot, const double* fadj, const double* U,
                                                      Phys ph, Terms extra, double* lamU) {
-    const AdjTile t = ld_const(tiles, blockIdx.x);
+    const AdjItem t = ld_const(tiles, tile_pos());
     if ((int)threadIdx.x >= t.count) return;
-    const DevBlock B = ld_const(blocks, t.block);  // descriptor in scalar registers
+    const DevBlock& B = t.b;  // in scalar registers
     const int e = t.start + threadIdx.x;
     const int k = e / B.nx, j = e - k * B.nx;
     Q4 lam = (B.kind == PHX_GEOM_CARTESIAN)
-                 ? phx::adj::gather_adj<true, NQ>(blocks, offs, t.block, k, j, slot, fadj, U, ph)
-                 : phx::adj::gather_adj<false, NQ>(blocks, offs, t.block, k, j, slot, fadj, U, ph);
+                 ? phx::adj::gather_adj_at<true, NQ>(blocks, offs, B, t.o, k, j, slot, fadj, U, ph)
+                 : phx::adj::gather_adj_at<false, NQ>(blocks, offs, B, t.o, k, j, slot, fadj, U, ph);
     if (extra.n > 0) phx::adj::acc(lam, eval_terms(extra, B, B.off / 4 + (long long)k * B.nx + j));
     phx::adj::st(lamU + B.off + 4LL * ((long long)k * B.nx + j), lam);
 }
 
 // ---- tangent-linear products (forward mode): three element-wise passes on the same tiles ----
-//   k_tan_recon   face states of every cell and their derivatives (16 + 16 doubles)
+//   k_tan_recon   face states of every cell and their derivatives (16 + 16 doubles; k_tan_recon_v with
+//                 one lane per cell and variable)
 //   k_tan_face    derivative of every face flux (4 doubles)
-//   k_tan_cell    derivative of every cell's residual (the residual is linear in the fluxes)
-__global__ void __launch_bounds__(TILE) k_tan_recon(const DevBlock* blocks, const AdjBlock* offs, const AdjTile* tiles,
+//   k_tan_cell    derivative of every cell's residual (the residual is linear in the fluxes) and what a
+//                 Runge-Kutta stage makes of it
+__global__ void __launch_bounds__(TILE) k_tan_recon(const DevBlock* blocks, const AdjBlock* offs, const AdjItem* tiles,
                                                     const double* U, const double* dU, double* rb, double* tb,
                                                     Phys ph) {
-    const AdjTile t = ld_const(tiles, blockIdx.x);
+    const AdjItem t = ld_const(tiles, tile_pos());
     if ((int)threadIdx.x >= t.count) return;
-    const DevBlock B = ld_const(blocks, t.block);  // descriptor in scalar registers
-    const AdjBlock O = ld_const(offs, t.block);
+    const DevBlock& B = t.b;  // in scalar registers
+    const AdjBlock& O = t.o;
     const int e = t.start + threadIdx.x;
     const int k = e / B.nx, j = e - k * B.nx;
     const long long c = phx::adj::RB * phx::adj::cell_index(O, B, k, j);
@@ -180,14 +215,30 @@ __global__ void __launch_bounds__(TILE) k_tan_recon(const DevBlock* blocks, cons
     else phx::tng::recon_cell_d<false>(blocks, B, U, dU, k, j, rb + c, tb + c, ph);
 }
 
+// Conservative reconstruction: one lane per cell and variable, as k_adj_recon_v.
+__global__ void __launch_bounds__(TILE) k_tan_recon_v(const DevBlock* blocks, const AdjBlock* offs,
+                                                       const AdjItem* tiles, const double* U, const double* dU,
+                                                       double* rb, double* tb, Phys ph) {
+    int c, v;
+    const AdjItem t = part_tile(tiles, c, v);
+    if (c >= t.count) return;
+    const DevBlock& B = t.b;  // in scalar registers
+    const AdjBlock& O = t.o;
+    const int e = t.start + c;
+    const int k = e / B.nx, j = e - k * B.nx;
+    const long long at = phx::adj::RB * phx::adj::cell_index(O, B, k, j);
+    if (B.kind == PHX_GEOM_CARTESIAN) phx::tng::recon_cell_var_d<true>(blocks, B, U, dU, k, j, v, rb + at, tb + at, ph);
+    else phx::tng::recon_cell_var_d<false>(blocks, B, U, dU, k, j, v, rb + at, tb + at, ph);
+}
+
 template <int FLUX>
-__global__ void __launch_bounds__(TILE) k_tan_face(const DevBlock* blocks, const AdjBlock* offs, const AdjTile* tiles,
+__global__ void __launch_bounds__(TILE) k_tan_face(const DevBlock* blocks, const AdjBlock* offs, const AdjItem* tiles,
                                                    const double* U, const double* dU, const double* rb,
                                                    const double* tb, double* dF, Phys ph) {
-    const AdjTile t = ld_const(tiles, blockIdx.x);
+    const AdjItem t = ld_const(tiles, tile_pos());
     if ((int)threadIdx.x >= t.count) return;
-    const DevBlock B = ld_const(blocks, t.block);  // descriptor in scalar registers
-    const AdjBlock O = ld_const(offs, t.block);
+    const DevBlock& B = t.b;  // in scalar registers
+    const AdjBlock& O = t.o;
     const long long f = (long long)t.start + threadIdx.x;
     const Q4 d = (B.kind == PHX_GEOM_CARTESIAN)
                      ? phx::tng::face_flux_d<true, FLUX>(blocks, B, U, dU, rb, tb, O, f, ph)
@@ -195,27 +246,29 @@ __global__ void __launch_bounds__(TILE) k_tan_face(const DevBlock* blocks, const
     phx::adj::st(dF + 4 * (O.face + f), d);
 }
 
-__global__ void __launch_bounds__(TILE) k_tan_cell(const DevBlock* blocks, const AdjBlock* offs, const AdjTile* tiles,
-                                                   const double* dF, double* out) {
-    const AdjTile t = ld_const(tiles, blockIdx.x);
+// K = residual derivative of the stage, stored if a later stage or the caller takes it (K not null), and
+// with Terms the next stage's input or the step's output: sum of the terms and ck * dt * K, at every cell
+__global__ void __launch_bounds__(TILE) k_tan_cell(const DevBlock* blocks, const AdjBlock* offs, const AdjItem* tiles,
+                                                   const double* dF, double* K, Terms terms, double ck, double* out) {
+    const AdjItem t = ld_const(tiles, tile_pos());
     if ((int)threadIdx.x >= t.count) return;
-    const DevBlock B = ld_const(blocks, t.block);  // descriptor in scalar registers
-    const AdjBlock O = ld_const(offs, t.block);
+    const DevBlock& B = t.b;  // in scalar registers
+    const AdjBlock& O = t.o;
     const int e = t.start + threadIdx.x;
     const int k = e / B.nx, j = e - k * B.nx;
+    const long long cell = B.off / 4 + e;
+    Q4 sum = phx::q4zero();
+    if (out) sum = eval_terms(terms, B, cell);
     const Q4 r = (B.kind == PHX_GEOM_CARTESIAN) ? phx::adj::cell_residual<true>(B, O, dF, k, j)
                                                 : phx::adj::cell_residual<false>(B, O, dF, k, j);
-    phx::adj::st(out + B.off + 4LL * ((long long)k * B.nx + j), r);
-}
-
-// out = sum of terms at every cell (the stage combinations of the tangent step)
-__global__ void __launch_bounds__(TILE) k_tan_combine(const DevBlock* blocks, const AdjTile* tiles, Terms terms,
-                                                      double* out) {
-    const AdjTile t = ld_const(tiles, blockIdx.x);
-    if ((int)threadIdx.x >= t.count) return;
-    const DevBlock B = ld_const(blocks, t.block);  // descriptor in scalar registers
-    const long long cell = B.off / 4 + t.start + threadIdx.x;
-    phx::adj::st(out + 4 * cell, eval_terms(terms, B, cell));
+    if (K) phx::adj::st(K + 4 * cell, r);
+    if (!out) return;
+    if (ck != 0.0) {
+        const double c = ck * terms.dt[B.case_id];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) sum.v[q] += c * r.v[q];
+    }
+    phx::adj::st(out + 4 * cell, sum);
 }
 
 template <class T>
@@ -264,8 +317,13 @@ int adj_meta(phx_plan* P) {
     P->adj_faces = faces;
     int rc;
     if ((rc = upload(offs, &P->dadj))) return rc;
-    if ((rc = upload(P->adj_cell_tiles, &P->dadj_cell_tiles))) return rc;
-    if ((rc = upload(P->adj_face_tiles, &P->dadj_face_tiles))) return rc;
+    auto items = [&](const std::vector<AdjTile>& tiles) {
+        std::vector<AdjItem> full;
+        for (const AdjTile& t : tiles) full.push_back({t.block, t.start, t.count, P->hblocks[t.block], offs[t.block]});
+        return full;
+    };
+    if ((rc = upload(items(P->adj_cell_tiles), &P->dadj_cell_tiles))) return rc;
+    if ((rc = upload(items(P->adj_face_tiles), &P->dadj_face_tiles))) return rc;
     P->adj_meta_ready = true;
     return PHX_OK;
 }
@@ -310,20 +368,26 @@ int tan_setup(phx_plan* P) {
     return PHX_OK;
 }
 
-void launch_residual_jvp(phx_plan* P, const double* U, const double* dU, double* out, hipStream_t st) {
+void launch_residual_jvp(phx_plan* P, const double* U, const double* dU, double* K, const Terms& terms, double ck,
+                         double* out, hipStream_t st) {
     const dim3 blk(TILE);
     const dim3 gc((unsigned)P->adj_cell_tiles.size()), gf((unsigned)P->adj_face_tiles.size());
     // face states in adj_rb, their derivatives in adj_slot (RB of its SLOT doubles per cell), face
     // flux derivatives in adj_face (4 of its FA doubles per face)
-    hipLaunchKernelGGL(k_tan_recon, gc, blk, 0, st, P->dblocks, P->dadj, P->dadj_cell_tiles, U, dU, P->adj_rb,
-                       P->adj_slot, P->ph);
+    if (P->ph.prim)
+        hipLaunchKernelGGL(k_tan_recon, gc, blk, 0, st, P->dblocks, P->dadj, P->dadj_cell_tiles, U, dU, P->adj_rb,
+                           P->adj_slot, P->ph);
+    else
+        hipLaunchKernelGGL(k_tan_recon_v, dim3(gc.x * VPARTS), blk, 0, st, P->dblocks, P->dadj, P->dadj_cell_tiles, U, dU,
+                           P->adj_rb, P->adj_slot, P->ph);
     if (P->flux == PHX_FLUX_ROE)
         hipLaunchKernelGGL(k_tan_face<0>, gf, blk, 0, st, P->dblocks, P->dadj, P->dadj_face_tiles, U, dU, P->adj_rb,
                            P->adj_slot, P->adj_face, P->ph);
     else
         hipLaunchKernelGGL(k_tan_face<1>, gf, blk, 0, st, P->dblocks, P->dadj, P->dadj_face_tiles, U, dU, P->adj_rb,
                            P->adj_slot, P->adj_face, P->ph);
-    hipLaunchKernelGGL(k_tan_cell, gc, blk, 0, st, P->dblocks, P->dadj, P->dadj_cell_tiles, P->adj_face, out);
+    hipLaunchKernelGGL(k_tan_cell, gc, blk, 0, st, P->dblocks, P->dadj, P->dadj_cell_tiles, P->adj_face, K,
+                       terms, ck, out);
 }
 
 int tan_check(phx_plan* P) {
@@ -364,10 +428,10 @@ double* scratch_of(int device) {
 template <int NQ>
 void launch_residual_vjp_nq(phx_plan* P, const double* U, const Terms& kappa, const Terms& extra, double* lamU,
                             const AdjBufs& w, hipStream_t st) {
-    const dim3 blk(TILE), vblk(VTILE);
-    const dim3 gc((unsigned)P->adj_cell_tiles.size()), gf((unsigned)P->adj_face_tiles.size());
+    const dim3 blk(TILE);
+    const dim3 gc((unsigned)P->adj_cell_tiles.size()), gv(gc.x * VPARTS), gf((unsigned)P->adj_face_tiles.size());
     if (NQ == 1)
-        hipLaunchKernelGGL(k_adj_recon_v, gc, vblk, 0, st, P->dblocks, P->dadj, P->dadj_cell_tiles, U, w.rb, P->ph);
+        hipLaunchKernelGGL(k_adj_recon_v, gv, blk, 0, st, P->dblocks, P->dadj, P->dadj_cell_tiles, U, w.rb, P->ph);
     else
         hipLaunchKernelGGL(k_adj_recon<NQ>, gc, blk, 0, st, P->dblocks, P->dadj, P->dadj_cell_tiles, U, w.rb,
                            P->ph);
@@ -378,7 +442,7 @@ void launch_residual_vjp_nq(phx_plan* P, const double* U, const Terms& kappa, co
         hipLaunchKernelGGL((k_adj_face<1, NQ>), gf, blk, 0, st, P->dblocks, P->dadj, P->dadj_face_tiles, U, w.rb,
                            kappa, w.face, P->ph);
     if (NQ == 1)
-        hipLaunchKernelGGL(k_adj_cell_v, gc, vblk, 0, st, P->dblocks, P->dadj, P->dadj_cell_tiles, U, w.face,
+        hipLaunchKernelGGL(k_adj_cell_v, gv, blk, 0, st, P->dblocks, P->dadj, P->dadj_cell_tiles, U, w.face,
                            w.slot, P->ph);
     else
         hipLaunchKernelGGL(k_adj_cell<NQ>, gc, blk, 0, st, P->dblocks, P->dadj, P->dadj_cell_tiles, U, w.face,
@@ -526,7 +590,9 @@ int phx_residual_jvp(phx_plan* P, const double* U, const double* dU, double* dR,
     if (!P || !U || !dU || !dR) return fail(PHX_E_INVALID, "null argument");
     int rc = tan_check(P);
     if (rc) return rc;
-    launch_residual_jvp(P, U, dU, dR, (hipStream_t)stream);
+    Terms none;
+    memset(&none, 0, sizeof(none));
+    launch_residual_jvp(P, U, dU, dR, none, 0.0, nullptr, (hipStream_t)stream);
     PHX_CK(hipGetLastError());
     return PHX_OK;
 }
@@ -543,12 +609,11 @@ int phx_step_jvp(phx_plan* P, const double* stages, const double* dt_dev, double
     const double* a = P->butcher.data();
     const dim3 gc((unsigned)P->adj_cell_tiles.size());
     for (int s = 0; s < S; ++s) {
-        launch_residual_jvp(P, stages + (size_t)s * L, s == 0 ? dU : P->tan_u, P->tan_k[s], st);
         Terms T;
         memset(&T, 0, sizeof(T));
         T.in[T.n] = dU;
         T.c[T.n++] = 1.0;
-        for (int m = 0; m <= s; ++m) {
+        for (int m = 0; m < s; ++m) {
             const double c = a[(size_t)s * S + m];
             if (c == 0.0) continue;
             T.in[T.n] = P->tan_k[m];
@@ -556,8 +621,10 @@ int phx_step_jvp(phx_plan* P, const double* stages, const double* dt_dev, double
             T.scaled[T.n++] = 1;
         }
         T.dt = dt_dev;
-        hipLaunchKernelGGL(k_tan_combine, gc, dim3(TILE), 0, st, P->dblocks, P->dadj_cell_tiles, T,
-                           s + 1 < S ? P->tan_u : dU);
+        bool later = false;
+        for (int l = s + 1; l < S; ++l) later = later || a[(size_t)l * S + s] != 0.0;
+        launch_residual_jvp(P, stages + (size_t)s * L, s == 0 ? dU : P->tan_u, later ? P->tan_k[s] : nullptr, T,
+                            a[(size_t)s * S + s], s + 1 < S ? P->tan_u : dU, st);
     }
     PHX_CK(hipGetLastError());
     return PHX_OK;

@@ -71,6 +71,17 @@ __host__ __device__ inline bool is_zero(const Q4& a) {
     return a.v[0] == 0.0 && a.v[1] == 0.0 && a.v[2] == 0.0 && a.v[3] == 0.0;
 }
 
+// The values are wanted here: their loads are not moved behind a later branch, where they would begin a
+// second round trip to memory.
+__host__ __device__ inline void wanted(double& x) {
+#ifdef __HIP_DEVICE_COMPILE__
+    asm volatile("" : "+v"(x));
+#endif
+}
+__host__ __device__ inline void wanted(Q4& q) {
+    wanted(q.v[0]); wanted(q.v[1]); wanted(q.v[2]); wanted(q.v[3]);
+}
+
 // ---------------------------------------------------------------------------------------------
 // pass 1: limited face states of cell (k, j) (the reconstruction of the stage kernel); the
 // variables are independent, and the device runs one lane per cell and variable
@@ -125,7 +136,8 @@ __host__ __device__ inline void recon_cell_var(const DevBlock* blocks, const Dev
     const double un = fetch_var<CART>(blocks, B, U, k + 1, j, v, ph);
     const CellGeo g = dev::cell_geo<CART>(B, k, j);
     double qE, qW, qN, qS;
-    reconstruct_var<true>(u, uw, ue, us, un, g, ph.limiter, qE, qW, qN, qS);
+    if (ph.limiter == PHX_LIMITER_VENKATAKRISHNAN) reconstruct_var<false>(u, uw, ue, us, un, g, ph.limiter, qE, qW, qN, qS);
+    else reconstruct_var<true>(u, uw, ue, us, un, g, ph.limiter, qE, qW, qN, qS);
     rb[RB_E + v] = qE;
     rb[RB_W + v] = qW;
     rb[RB_N + v] = qN;
@@ -432,7 +444,14 @@ template <bool CART>
 __host__ __device__ inline void cell_adj_var(const DevBlock* blocks, const DevBlock& B, const double* U,
                                              const AdjBlock& O, const double* fadj, int k, int j, int v, double* slot,
                                              const Phys& ph) {
+    // every load first: what bounds this pass is the latency of memory, not its few waves' arithmetic
     const int nx = B.nx, ny = B.ny;
+    double u = fetch_var<CART>(blocks, B, U, k, j, v, ph);
+    double uw = fetch_var<CART>(blocks, B, U, k, j - 1, v, ph);
+    double ue = fetch_var<CART>(blocks, B, U, k, j + 1, v, ph);
+    double us = fetch_var<CART>(blocks, B, U, k - 1, j, v, ph);
+    double un = fetch_var<CART>(blocks, B, U, k + 1, j, v, ph);
+    const CellGeo g = dev::cell_geo<CART>(B, k, j);
     double bq[4] = {fadj[FA * xface_index(O, B, k, j + 1) + v], fadj[FA * xface_index(O, B, k, j) + 4 + v],
                     fadj[FA * yface_index(O, B, k + 1, j) + v], fadj[FA * yface_index(O, B, k, j) + 4 + v]};
     if (j == nx - 1) bq[0] += comp(outer_own_adj<CART>(B, PHX_E, ld(fadj + FA * xface_index(O, B, k, nx) + 4), k, nx), v);
@@ -440,16 +459,10 @@ __host__ __device__ inline void cell_adj_var(const DevBlock* blocks, const DevBl
     if (k == ny - 1)
         bq[2] += comp(outer_own_adj<CART>(B, PHX_N, ld(fadj + FA * yface_index(O, B, ny, j) + 4), ny - 1, j), v);
     if (k == 0) bq[3] += comp(outer_own_adj<CART>(B, PHX_S, ld(fadj + FA * yface_index(O, B, 0, j)), 0, j), v);
+    wanted(u); wanted(uw); wanted(ue); wanted(us); wanted(un);
     double o[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    if (bq[0] != 0.0 || bq[1] != 0.0 || bq[2] != 0.0 || bq[3] != 0.0) {
-        const double u = fetch_var<CART>(blocks, B, U, k, j, v, ph);
-        const double uw = fetch_var<CART>(blocks, B, U, k, j - 1, v, ph);
-        const double ue = fetch_var<CART>(blocks, B, U, k, j + 1, v, ph);
-        const double us = fetch_var<CART>(blocks, B, U, k - 1, j, v, ph);
-        const double un = fetch_var<CART>(blocks, B, U, k + 1, j, v, ph);
-        const CellGeo g = dev::cell_geo<CART>(B, k, j);
+    if (bq[0] != 0.0 || bq[1] != 0.0 || bq[2] != 0.0 || bq[3] != 0.0)
         reconstruct_vjp_var(u, uw, ue, us, un, g, bq, ph.limiter, o);
-    }
     slot[SL_C + v] = o[0];
     slot[SL_W + v] = o[1];
     slot[SL_E + v] = o[2];
@@ -476,10 +489,9 @@ __host__ __device__ inline Q4 wall_ghost_adj(const DevBlock& B, int side, const 
 // conversion to primitive variables once; a wall ghost is the reflected state converted, and is
 // taken back on its own.
 template <bool CART, int NQ = 1>
-__host__ __device__ inline Q4 gather_adj(const DevBlock* blocks, const AdjBlock* offs, int b, int k, int j,
-                                         const double* slot, const double* fadj, const double* U, const Phys& ph) {
-    const DevBlock& B = blocks[b];
-    const AdjBlock& O = offs[b];
+__host__ __device__ inline Q4 gather_adj_at(const DevBlock* blocks, const AdjBlock* offs, const DevBlock& B,
+                                            const AdjBlock& O, int k, int j, const double* slot, const double* fadj,
+                                            const double* U, const Phys& ph) {
     const int nx = B.nx, ny = B.ny;
     const int nq = npts<NQ>(ph);
     // adjoint of a boundary face's outer state that is a ghost cell value, summed over the face's
@@ -550,6 +562,11 @@ __host__ __device__ inline Q4 gather_adj(const DevBlock* blocks, const AdjBlock*
     if (ph.prim) lam = cons_to_prim_vjp(q, PrimBar{own.v[0], own.v[1], own.v[2], own.v[3]}, ph);
     acc(lam, walls);
     return lam;
+}
+template <bool CART, int NQ = 1>
+__host__ __device__ inline Q4 gather_adj(const DevBlock* blocks, const AdjBlock* offs, int b, int k, int j,
+                                         const double* slot, const double* fadj, const double* U, const Phys& ph) {
+    return gather_adj_at<CART, NQ>(blocks, offs, blocks[b], offs[b], k, j, slot, fadj, U, ph);
 }
 
 }  // namespace adj

@@ -137,6 +137,26 @@ __host__ __device__ inline void recon_cell_d(const dev::DevBlock* blocks, const 
     adj::st(tb + adj::RB_S, der(r.S));
 }
 
+// recon_cell_d for variable v only (conservative reconstruction, whose variables are independent): the four
+// calls v = 0..3 write exactly what recon_cell_d writes (one lane per cell and variable).
+template <bool CART>
+__host__ __device__ inline void recon_cell_var_d(const dev::DevBlock* blocks, const dev::DevBlock& B, const double* U,
+                                                 const double* dU, int k, int j, int v, double* rb, double* tb,
+                                                 const Phys& ph) {
+    auto at = [&](int kk, int jj) {
+        return D(adj::fetch_var<CART>(blocks, B, U, kk, jj, v, ph), adj::fetch_var<CART>(blocks, B, dU, kk, jj, v, ph));
+    };
+    const D u = at(k, j), uw = at(k, j - 1), ue = at(k, j + 1), us = at(k - 1, j), un = at(k + 1, j);
+    const CellGeo g = dev::cell_geo<CART>(B, k, j);
+    D q[4];
+    if (ph.limiter == PHX_LIMITER_VENKATAKRISHNAN) reconstruct_var<false>(u, uw, ue, us, un, g, ph.limiter, q[0], q[1], q[2], q[3]);
+    else reconstruct_var<true>(u, uw, ue, us, un, g, ph.limiter, q[0], q[1], q[2], q[3]);
+    for (int f = 0; f < 4; ++f) {
+        rb[4 * f + v] = q[f].v;
+        tb[4 * f + v] = q[f].d;
+    }
+}
+
 __host__ __device__ inline QD ld_d(const double* rb, const double* tb, long long cell, int off) {
     return make(adj::ld(rb + adj::RB * cell + off), adj::ld(tb + adj::RB * cell + off));
 }
