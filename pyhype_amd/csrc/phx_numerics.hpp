@@ -1160,10 +1160,33 @@ __host__ __device__ inline void reconstruct_q_var(double u, double uw, double ue
     const double s = 0.5 * (us + u);
     gx = (e * g.xlE + w * g.xlW + n * g.xlN + s * g.xlS) * g.ainv;
     gy = (e * g.ylE + w * g.ylW + n * g.ylN + s * g.ylS) * g.ainv;
-    const double mx = fmax(fmax(fmax(fmax(u, uw), ue), us), un);
-    const double mn = fmin(fmin(fmin(fmin(u, uw), ue), us), un);
+    const double mx = vmax(vmax(vmax(vmax(u, uw), ue), us), un);
+    const double mn = vmin(vmin(vmin(vmin(u, uw), ue), us), un);
     const double dmax = mx - u;
     const double dmin = mn - u;
+    if (lim == 1) {
+        // Barth-Jespersen: min(1, slope) rises with the slope and division rounds monotonically, so the smallest
+        // slopes are dmax / max(d) and dmin / min(d): 2 divisions instead of one per point, the same bits.
+        // Values and gradient of at most 2^600 and geometry of at most 2^60 leave no infinity or NaN among
+        // the d; with both extrema at the cell the sign of the zero depends on the points' order.
+        double P = 0.0, M = 0.0;
+#pragma unroll
+        for (int f = 0; f < 4; ++f)
+#pragma unroll
+            for (int i = 0; i < QMAX; ++i) {
+                if (i >= nq) continue;
+                const double d = (u + (gx * q.dx[f][i] + gy * q.dy[f][i])) - u;
+                P = vmax(P, d);
+                M = vmin(M, d);
+            }
+        const int usual = (fabs(gx) <= 0x1p600) & (fabs(gy) <= 0x1p600) & (fabs(u) <= 0x1p600) & (dmax - dmin <= 0x1p600) &
+                          !((dmax == 0.0) & (dmin == 0.0) & (P > M));
+        if (PHX_USUAL(!g.odd && wave_all(usual))) {
+            const double sP = (P > 0.0) ? dmax / P : 1.0, sM = (M < 0.0) ? dmin / M : 1.0;
+            phi = vmin(vmin(sP, sM), 1.0);
+            return;
+        }
+    }
     double p = 0.0;
 #pragma unroll
     for (int f = 0; f < 4; ++f)

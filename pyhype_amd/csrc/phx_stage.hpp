@@ -854,8 +854,7 @@ __device__ __forceinline__ void acc_w(Q4& acc, double w, const Q4& F) {
 
 template <bool CART, int FLUX>
 __device__ __forceinline__ void recon_x_item_q(const StageArgs& A, const DevItem& it) {
-    const DevBlock& B = A.blocks[it.block];
-    if (frozen_case(A, B)) return;
+    const DevBlock& B = it.b;
     const int nx = B.nx;
     const int j = it.j0 - HALO + threadIdx.x % WAVE;
     const bool valid = (j >= -1) && (j <= nx);
@@ -873,18 +872,24 @@ __device__ __forceinline__ void recon_x_item_q(const StageArgs& A, const DevItem
     for (int k = it.r0; k < it.r1; ++k) {
         if (inner) Up = fetch_r<CART, true>(A.blocks, B, A.Uin, k + 1, j, ph);
         else if (gcol && k + 1 < it.r1) Up = fetch_r<CART, true>(A.blocks, B, A.Uin, k + 1, j, ph);
+        // the row's loads before its arithmetic: this stage waits for memory half of its time
+        phx::CellGeo g;
+        phx::QGeo qg;
+        double LW = 0.0, LE = 0.0, LS, LN, Ac;
+        if (recon) {
+            g = cell_geo<CART>(B, k, j);
+            qg = cell_qgeo(B, k, j, nq);
+        } else {
+            for (int f = 0; f < 4; ++f)
+                for (int i = 0; i < phx::QMAX; ++i) qg.dx[f][i] = qg.dy[f][i] = 0.0;
+        }
+        if (owner) cell_L<CART>(B, k, j, LW, LE, LS, LN, Ac);
+        if (frozen_case(A, B)) return;
         const Q4 Uw = shfl_up1(Uc);
         const Q4 Ue = shfl_down1(Uc);
         phx::ReconQ r;
         r.u = r.gx = r.gy = r.phi = phx::q4zero();
-        phx::QGeo qg;
-        for (int f = 0; f < 4; ++f)
-            for (int i = 0; i < phx::QMAX; ++i) qg.dx[f][i] = qg.dy[f][i] = 0.0;
-        if (recon) {
-            const phx::CellGeo g = cell_geo<CART>(B, k, j);
-            qg = cell_qgeo(B, k, j, nq);
-            r = phx::reconstruct_q(Uc, Uw, Ue, Um, Up, g, qg, nq, ph.limiter);
-        }
+        if (recon) r = phx::reconstruct_q(Uc, Uw, Ue, Um, Up, g, qg, nq, ph.limiter);
         Q4 SW = phx::q4zero();  // sum over the W face's points of w_i * F_i
 #pragma unroll
         for (int i = 0; i < phx::QMAX; ++i) {
@@ -900,8 +905,6 @@ __device__ __forceinline__ void recon_x_item_q(const StageArgs& A, const DevItem
         }
         const Q4 SE = shfl_down1(SW);
         if (owner) {
-            double LW, LE, LS, LN, Ac;
-            cell_L<CART>(B, k, j, LW, LE, LS, LN, Ac);
             Q4 part;
 #pragma unroll
             for (int c = 0; c < 4; ++c) part.v[c] = LW * SW.v[c] - LE * SE.v[c];
