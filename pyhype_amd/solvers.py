@@ -97,11 +97,15 @@ def validate_config(config) -> List[List[float]]:
 #    of neighbouring rows meet in one L2 (8 x 10^5: 94.1 against 99.6).
 #  * The fused stage beyond, with items of 8 rows or more (1.1 x 10^6 cells: 4 rows 111.9, 8 rows 96.2;
 #    2.4 x 10^6: 4 rows 221.6, 10 rows 201.0).
+#  * More than one Gauss point per face: strips, one row per item (two take 110 to 2 % longer from 40^2 to
+#    800 x 600 cells), with 1, 2 or 3 rows of the update (two points, 100^2: 18.8, 23.0, 23.0; 200 x 120: 22.3,
+#    20.8, 21.7; 800 x 600: 99.8, 93.4, 91.0).
 SHARED_ITEMS = (256, 384)          # workgroups of the shared-halo stage with 1 and 2 rows
 STRIP_CELLS = 100_000
 DEALT_CELLS = 250_000
 SPLIT_CELLS = {"Roe": 1_000_000, "HLLL": 2_500_000}
 FUSED_ROWS = 8
+GAUSS_CELLS = (16_000, 100_000)    # up to which the update of a plan with Gauss points takes 1 and 2 rows
 
 
 def default_rows(cells: int) -> int:
@@ -112,8 +116,9 @@ def default_rows(cells: int) -> int:
 def default_shape(plan) -> dict:
     """``DevicePlan.set_launch`` arguments for a workload without a tuned shape (see above)."""
     cells = plan.cells()
-    if plan.quadrature_points > 1:   # the split stage of the plan; rows of a reconstruction item
-        return {"rows_per_item": 1 if cells < STRIP_CELLS else 2}
+    if plan.quadrature_points > 1:
+        return {"rows_per_item": 1, "waves_per_simd": 3, "variant": 6,
+                "rows_b": 1 if cells < GAUSS_CELLS[0] else (2 if cells < GAUSS_CELLS[1] else 3)}
     kinds = {e.cartesian for e in plan.blocks}
     strips = [(-(-e.nx // 60), e.ny) for e in plan.blocks]
     for rows, most in zip((1, 2), SHARED_ITEMS):

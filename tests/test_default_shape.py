@@ -28,6 +28,7 @@ def test_default_shape(p, variant, rows):
     assert shape.get("xcd_chunk", 0) == (64 if variant == 7 and p.cells() > solvers.DEALT_CELLS else 0)
 
 
-def test_default_shape_keeps_the_split_stage_of_more_gauss_points():
-    for n, rows in ((40, 1), (400, 2)):
-        assert solvers.default_shape(plan([(n, n)], nq=2)) == {"rows_per_item": rows}
+@pytest.mark.parametrize("n, rows_b", [(1, 1), (126, 1), (127, 2), (316, 2), (317, 3), (3000, 3)])
+def test_default_shape_of_more_gauss_points(n, rows_b):
+    shape = solvers.default_shape(plan([(n, n)], nq=2))
+    assert (shape["variant"], shape["rows_per_item"], shape["rows_b"]) == (6, 1, rows_b)
