@@ -1179,8 +1179,8 @@ __host__ __device__ inline void reconstruct_q_var(double u, double uw, double ue
                 P = vmax(P, d);
                 M = vmin(M, d);
             }
-        const int usual = (fabs(gx) <= 0x1p600) & (fabs(gy) <= 0x1p600) & (fabs(u) <= 0x1p600) & (dmax - dmin <= 0x1p600) &
-                          !((dmax == 0.0) & (dmin == 0.0) & (P > M));
+        const int usual = (int)(fabs(gx) <= 0x1p600) & (fabs(gy) <= 0x1p600) & (fabs(u) <= 0x1p600) & (dmax - dmin <= 0x1p600) &
+                          !((int)(dmax == 0.0) & (dmin == 0.0) & (P > M));
         if (PHX_USUAL(!g.odd && wave_all(usual))) {
             const double sP = (P > 0.0) ? dmax / P : 1.0, sM = (M < 0.0) ? dmin / M : 1.0;
             phi = vmin(vmin(sP, sM), 1.0);
