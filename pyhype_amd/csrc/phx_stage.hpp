@@ -170,7 +170,11 @@ __device__ __forceinline__ bool fold_step(const StageArgs& A) {
     return true;
 }
 
-// cross-lane moves of a 4-vector
+// Cross-lane moves of a 4-vector by one lane (the end lanes keep their value), in two forms: through the
+// LDS pipe (ds_bpermute_b32), and as v_mov_b32 with a wave shift, two to a double.  The first leaves the
+// vector pipe to the arithmetic that bounds the fused stage (batch of 2.4 x 10^6 cells, 8 steps: 6,423
+// us, with shifts 6,772); the second has no latency for a wave to wait out, which is what the split
+// stage's reconstruction does (5 x 500^2 HLLL, 16 steps: 3,088 us, with shifts 3,025).
 __device__ __forceinline__ Q4 shfl_up1(const Q4& q) {
     Q4 r;
 #pragma unroll
@@ -183,6 +187,21 @@ __device__ __forceinline__ Q4 shfl_down1(const Q4& q) {
     for (int k = 0; k < 4; ++k) r.v[k] = __shfl_down(q.v[k], 1, WAVE);
     return r;
 }
+template <int CTRL>
+__device__ __forceinline__ Q4 wave_shift(const Q4& q) {
+    Q4 r;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const unsigned long long b = __builtin_bit_cast(unsigned long long, q.v[k]);
+        const int lo = (int)(unsigned)b, hi = (int)(unsigned)(b >> 32);
+        const unsigned l = (unsigned)__builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xf, 0xf, false);
+        const unsigned h = (unsigned)__builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xf, 0xf, false);
+        r.v[k] = __builtin_bit_cast(double, ((unsigned long long)h << 32) | l);
+    }
+    return r;
+}
+__device__ __forceinline__ Q4 shift_up1(const Q4& q) { return wave_shift<0x138>(q); }    // wave_shr:1
+__device__ __forceinline__ Q4 shift_down1(const Q4& q) { return wave_shift<0x130>(q); }  // wave_shl:1
 
 // Outputs of the stage program are written in chunks of EMIT_CHUNK: the chunk's sources are loaded
 // together before its stores (an output's source is never a buffer an earlier output of the stage
@@ -885,8 +904,8 @@ __device__ __forceinline__ void recon_x_item_q(const StageArgs& A, const DevItem
         }
         if (owner) cell_L<CART>(B, k, j, LW, LE, LS, LN, Ac);
         if (frozen_case(A, B)) return;
-        const Q4 Uw = shfl_up1(Uc);
-        const Q4 Ue = shfl_down1(Uc);
+        const Q4 Uw = shift_up1(Uc);
+        const Q4 Ue = shift_down1(Uc);
         phx::ReconQ r;
         r.u = r.gx = r.gy = r.phi = phx::q4zero();
         if (recon) r = phx::reconstruct_q(Uc, Uw, Ue, Um, Up, g, qg, nq, ph.limiter);
@@ -895,7 +914,7 @@ __device__ __forceinline__ void recon_x_item_q(const StageArgs& A, const DevItem
         for (int i = 0; i < phx::QMAX; ++i) {
             if (i >= nq) break;
             const Q4 qsend = (j == -1) ? Uc : phx::qstate(r, qg, PHX_E, i);
-            const Q4 QEl = shfl_up1(qsend);  // limited east state of cell j-1 at point i
+            const Q4 QEl = shift_up1(qsend);  // limited east state of cell j-1 at point i
             if (xface) {
                 const Q4 Wi = phx::qstate(r, qg, PHX_W, i);
                 const Q4 L = (j == 0) ? outer_state<CART>(B, PHX_W, Wi, QEl, k, j) : QEl;
@@ -903,7 +922,7 @@ __device__ __forceinline__ void recon_x_item_q(const StageArgs& A, const DevItem
                 acc_w(SW, phx::gauss_w(nq, i), xflux<CART, FLUX, true>(B, L, R, k, j, ph));
             }
         }
-        const Q4 SE = shfl_down1(SW);
+        const Q4 SE = shift_down1(SW);
         if (owner) {
             Q4 part;
 #pragma unroll
@@ -1015,22 +1034,22 @@ __device__ __forceinline__ void recon_x_item(const StageArgs& A, const DevItem& 
         if (recon) g = cell_geo<CART>(B, k, j);
         if (owner) cell_L<CART>(B, k, j, LW, LE, LS, LN, Ac);
         if (frozen_case(A, B)) return;
-        const Q4 Uw = shfl_up1(Uc);
-        const Q4 Ue = shfl_down1(Uc);
+        const Q4 Uw = shift_up1(Uc);
+        const Q4 Ue = shift_down1(Uc);
         phx::Recon r;
         r.E = r.W = r.N = r.S = phx::q4zero();
         if (recon) {
             r = phx::reconstruct<GEN>(Uc, Uw, Ue, Um, Up, g, ph.limiter);
         }
         const Q4 qsend = (j == -1) ? Uc : r.E;
-        const Q4 QEl = shfl_up1(qsend);  // limited east state of cell j-1 (ghost value for j == 0)
+        const Q4 QEl = shift_up1(qsend);  // limited east state of cell j-1 (ghost value for j == 0)
         Q4 FW = phx::q4zero();
         if (xface) {
             const Q4 L = (j == 0) ? outer_state<CART>(B, PHX_W, r.W, QEl, k, j) : QEl;
             const Q4 R = (j == nx) ? outer_state<CART>(B, PHX_E, QEl, Uc, k, j) : r.W;
             FW = xflux<CART, FLUX, GEN>(B, L, R, k, j, ph);
         }
-        const Q4 FE = shfl_down1(FW);
+        const Q4 FE = shift_down1(FW);
         if (owner) {
             Q4 part;
 #pragma unroll
@@ -1336,8 +1355,8 @@ __device__ __forceinline__ void recon_x_lin_item(const StageArgs& A, const DevIt
         cell_L<CART>(B, k, j, LW, LE, LS, LN, Ac);
     }
     if (frozen_case(A, B)) return;
-    const Q4 Uwl = shfl_up1(Uc);
-    const Q4 Uel = shfl_down1(Uc);
+    const Q4 Uwl = shift_up1(Uc);
+    const Q4 Uel = shift_down1(Uc);
     if (!wmem) Uw = Uwl;
     if (!emem) Ue = Uel;
     phx::Recon r;
@@ -1345,14 +1364,14 @@ __device__ __forceinline__ void recon_x_lin_item(const StageArgs& A, const DevIt
     if (cell) {
         r = phx::reconstruct<GEN>(Uc, Uw, Ue, Um, Up, g, ph.limiter);
     }
-    const Q4 QEl = shfl_up1(r.E);  // limited east state of position p-1 (cell j-1 of the same row for j > 0)
+    const Q4 QEl = shift_up1(r.E);  // limited east state of position p-1 (cell j-1 of the same row for j > 0)
     Q4 FW = phx::q4zero();
     if (valid && lane > 0) {
         const Q4 L = (j == 0) ? outer_state<CART>(B, PHX_W, r.W, Uw, k, j) : QEl;
         const Q4 R = (j == nx) ? outer_state<CART>(B, PHX_E, QEl, Uc, k, j) : r.W;
         FW = xflux<CART, FLUX, GEN>(B, L, R, k, j, ph);
     }
-    const Q4 FE = shfl_down1(FW);
+    const Q4 FE = shift_down1(FW);
     if (cell && lane > 0 && lane < WAVE - 1) {
         Q4 part;
 #pragma unroll
