@@ -998,10 +998,10 @@ int phx_run(phx_plan* P, double* U, int32_t nsteps, int32_t use_graph, void* str
     if (P->graph_U != U) release_graphs(P);
     // The largest graph while enough steps remain, then one graph for each bit of the rest, largest
     // first: every graph but the last starts after an even number of steps, so that one capture of each
-    // size fits the alternation of the minima.  Captured when first needed; later calls replay.
+    // size fits the alternation of the minima.  All captured on first use, so that later calls only replay.
     const int most = 1 << (GRAPHS - 1);
     for (int g = 0; g < GRAPHS; ++g) {
-        if (P->gexec[g] || !(g == GRAPHS - 1 ? nsteps >= most : (nsteps >> g) & 1)) continue;
+        if (P->gexec[g]) continue;
         PHX_CK(hipStreamBeginCapture(P->cap_stream, hipStreamCaptureModeThreadLocal));
         for (int s = 0; s < 1 << g; ++s) launch_step(P, U, P->cap_stream, nullptr, s);
         PHX_CK(hipStreamEndCapture(P->cap_stream, &P->graph[g]));

@@ -34,8 +34,8 @@ constexpr int STRIP = WAVE - 2 * HALO;  // owned columns per wavefront
 constexpr unsigned long long DT_INF_BITS = 0x7FF0000000000000ull;  // +inf
 // The CFL minimum of a case is accumulated in nslot partial minima (a power of two, at most
 // DT_SLOTS), each on a cache line of its own (DT_STRIDE words apart): the waves of a stage spread
-// their atomicMin over the slots instead of serialising on one address, and k_finalize takes the
-// minimum over the slots (an exact operation, independent of the order).  Plans with many cases
+// their atomicMin over the slots instead of serialising on one address, and step_dt or k_finalize takes
+// the minimum over the slots (an exact operation, independent of the order).  Plans with many cases
 // use fewer slots per case (their waves are spread over the cases already).
 constexpr int DT_SLOTS = 64;
 constexpr int DT_STRIDE = 16;
