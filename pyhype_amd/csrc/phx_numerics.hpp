@@ -1072,11 +1072,30 @@ __host__ __device__ __forceinline__ double limit_venkat(double u, double dmax, d
     const double x = limiter_min4<false>(pE, pW, pN, pS);
     return (x < 0.0) ? 0.0 : x;
 }
+// Barth-Jespersen's value of one variable of a cell, as limit_venkat: min(1, slope) rises with the slope and
+// division rounds monotonically, so the smallest slopes are dmax / max(d) and dmin / min(d) (2 divisions
+// instead of 4, the same bits).  Values and increments of at most 2^600 leave no infinity or NaN among the
+// d; with both extrema at the cell the sign of the zero depends on the faces' order.
+__host__ __device__ __forceinline__ double limit_bj(double u, double dmax, double dmin, const double (&h)[4]) {
+    const double dE = (u + h[0]) - u, dW = (u + h[1]) - u, dN = (u + h[2]) - u, dS = (u + h[3]) - u;
+    const double P = vmax(vmax(vmax(dE, dW), vmax(dN, dS)), 0.0), M = vmin(vmin(vmin(dE, dW), vmin(dN, dS)), 0.0);
+    const double size = fabs(u) + ((fabs(h[0]) + fabs(h[1])) + (fabs(h[2]) + fabs(h[3])));
+    const int usual = (int)(size <= 0x1p600) & (dmax - dmin <= 0x1p600) & !((int)(dmax == 0.0) & (dmin == 0.0) & (P > M));
+    if (PHX_USUAL(wave_all(usual))) {
+        const double sP = (P > 0.0) ? dmax / P : 1.0, sM = (M < 0.0) ? dmin / M : 1.0;
+        return vmin(vmin(sP, sM), 1.0);
+    }
+    const double pE = limit_face<true>(dmax, dmin, dE, 1), pW = limit_face<true>(dmax, dmin, dW, 1);
+    const double pN = limit_face<true>(dmax, dmin, dN, 1), pS = limit_face<true>(dmax, dmin, dS, 1);
+    const double phi = limiter_min4<true>(pE, pW, pN, pS);
+    return (phi < 0.0) ? 0.0 : phi;
+}
 // The general form: any scalar type, with GEN the limiter `lim`.
 template <bool GEN, class T>
 __host__ __device__ inline T limit_cell(const T& u, const T& dmax, const T& dmin, const T (&h)[4], bool odd, int lim) {
     if constexpr (std::is_same<T, double>::value) {
-        if (!GEN || lim == 0) return limit_venkat(u, dmax, dmin, h, odd);
+        if (PHX_USUAL(!GEN || lim == 0)) return limit_venkat(u, dmax, dmin, h, odd);
+        if (lim == 1) return limit_bj(u, dmax, dmin, h);
     }
     const T pE = limit_face<GEN>(dmax, dmin, (u + h[0]) - u, lim);
     const T pW = limit_face<GEN>(dmax, dmin, (u + h[1]) - u, lim);
