@@ -2,8 +2,8 @@
 
 Fused variant: the work item is a 60-column strip of one block over ``rows_per_item`` rows; each
 item recomputes one reconstruction row above and below its range, so short items waste work while
-long items leave SIMDs idle on small meshes.  Shared-halo variant: workgroups of 4 waves with
-``rows_per_item`` rows each exchange their boundary rows through LDS.  Split variant: a reconstruction kernel with no row
+long items leave SIMDs idle on small meshes.  Shared-halo variant: workgroups of 12 or 16 waves
+share the states and fluxes of 1 or 2 rows through LDS.  Split variant: a reconstruction kernel with no row
 halo (``rows_per_item`` rows per item) and a y-face kernel (``rows_b`` rows per item).
 Element-wise variant: one lane per cell and variable for the reconstruction, one per face for
 the fluxes and one per cell for the update (no shape parameters).  Paired variant: the fused
