@@ -73,9 +73,25 @@ class Trajectory:
                 P.run_frozen(dt, check=False)
             else:
                 P.run_record(dt, self.stages[:dt.shape[0]])
-                self._recorded = True
-        P.check_realizable()
+        bad, step, _, _ = P.status()
+        if (bad >= 0).any():
+            self._failed_states(bad, step)
+        P.check_realizable(bad)
+        self._recorded = self.nsteps > 0
         return P.U.clone()
+
+    def _failed_states(self, bad, step):
+        """Put the states that the status describes into ``plan.U``.  A recorded segment writes ``plan.U`` in
+        its last step only, which a case that failed before it skips: that case's state is the input that
+        its failing step recorded for the next one."""
+        P = self.plan
+        last = min(self.every, self.nsteps - (len(self.checkpoints) - 1) * self.every)
+        for c, b in enumerate(bad):
+            i = int(b) - (step - last)          # 1-based place of the failing step in the last segment
+            if b >= 0 and 0 < i < last:
+                for e in P.case_blocks[c].values():
+                    at = slice(e.offset, e.offset + 4 * e.nx * e.ny)
+                    P.U[at].copy_(self.stages[i, 0, at])
 
     def backward(self, lam_T):
         """Adjoint of U_0 from the adjoint of U_n (the checkpoints of the last forward).
