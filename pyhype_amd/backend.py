@@ -378,9 +378,10 @@ class DevicePlan:
 
     def set_launch(self, rows_per_item: int, grid_waves: int = 0, waves_per_simd: int = 2,
                    variant: Optional[int] = None, rows_b: int = 0, xcd_chunk: Optional[int] = None):
-        """Launch shape of the stage: rows per work item, persistent grid (0 = one wave per item),
-        register budget in waves per SIMD; optionally the stage variant (0 fused, 1 split, 2 shared
-        halo, 3 element-wise, 4 paired, 5 split with fused y-face/update, 6 the same with one face per
+        """Launch shape of the stage: rows per work item (2 or more are 2 in the shared-halo stage),
+        persistent grid (0 = one wave per item), register budget as a level of 2, 3 or 4 (the header says
+        how many waves per SIMD each kernel makes of it); optionally the stage variant (0 fused, 1 split,
+        2 shared halo, 3 element-wise, 4 paired, 5 split with fused y-face/update, 6 the same with one face per
         wave, 7 variant 6 with the row-major reconstruction kernel, 8 that reconstruction with the
         y-faces and update over flat cell ranges), the rows per item of the split variants' update kernel
         and the order of the split variants' work lists over the XCDs (0 contiguous ranges, k > 0
@@ -407,6 +408,8 @@ class DevicePlan:
         nat.check(self.lib.phx_launch_info(self.handle, *[C.byref(x) for x in v]), "phx_launch_info")
         out = {"items_cart": v[0].value, "items_gen": v[1].value, "grid_cart": v[2].value, "grid_gen": v[3].value}
         out.update(getattr(self, "launch", {}))
+        if out.get("variant") == 2:   # a workgroup of the shared-halo stage takes 1 or 2 rows
+            out["rows_per_item"] = min(out["rows_per_item"], 2)
         return out
 
     def cells(self) -> int:
