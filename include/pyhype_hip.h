@@ -232,8 +232,12 @@ int phx_residual_vjp_noalloc(phx_plan* plan, const double* U, const double* lamR
 int phx_step_vjp(phx_plan* plan, const double* stages, const double* dt_dev, double* lam, void* stream);
 
 /* Tunables of the stage launch: rows per work item, persistent grid size in waves (0 = one
- * workgroup per item) and the register budget variant (waves per SIMD, 2, 3 or 4; 0 = 2; the
- * fused kernel uses at most 3); rebuilds the work list.  Used by the autotuner in
+ * workgroup per item) and the register budget, a level of 2, 3 or 4 (0 = 2); rebuilds the work
+ * list.  Waves per SIMD that a kernel's registers allow at levels 2, 3 and 4: fused and paired
+ * stage 2, 3, 3; strip reconstruction (variants 1, 5, 6) 2, 2, 3; row-major reconstruction
+ * (variants 7, 8) 3, 3, 4 with Roe and 4, 4, 4 with HLLL (3, 3, 4 on a mesh of both geometry
+ * kinds in one launch).  With another limiter or primitive reconstruction the row-major kernel
+ * allows 3 at every level and the others 2.  The other kernels have one budget.  Used by the autotuner in
  * pyhype_amd/autotune.py.  No counterpart in the reference. */
 int phx_set_launch(phx_plan* plan, int32_t rows_per_item, int32_t grid_waves, int32_t waves_per_simd);
 

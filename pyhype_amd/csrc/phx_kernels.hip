@@ -478,8 +478,8 @@ StageArgs base_args(phx_plan* P) {
     return A;
 }
 
-// one launch of kernel family T over the items of one geometry kind; minw = register budget in
-// waves per SIMD (2, 3 or 4)
+// one launch of kernel family T over the items of one geometry kind; minw = register budget asked for
+// (2, 3 or 4)
 template <class T>
 void launch_kind(const phx_plan* P, StageArgs& S, int kind, const DevItem* items, int nitems, int grid, int minw,
                  hipStream_t st) {

@@ -174,7 +174,7 @@ __device__ __forceinline__ bool fold_step(const StageArgs& A) {
 // LDS pipe (ds_bpermute_b32), and as v_mov_b32 with a wave shift, two to a double.  The first leaves the
 // vector pipe to the arithmetic that bounds the fused stage (batch of 2.4 x 10^6 cells, 8 steps: 6,423
 // us, with shifts 6,772); the second has no latency for a wave to wait out, which is what the split
-// stage's reconstruction does (5 x 500^2 HLLL, 16 steps: 3,088 us, with shifts 3,025).
+// stage's reconstruction does (5 x 500^2 HLLL, 16 steps: 3,128 us, with shifts 3,059).
 __device__ __forceinline__ Q4 shfl_up1(const Q4& q) {
     Q4 r;
 #pragma unroll
@@ -1566,9 +1566,10 @@ __global__ void __launch_bounds__(EW_WG) k_ew_update(StageArgs A) {
 
 // Launchers of the stage kernel families, one per kernel template; each is defined in the translation
 // unit that instantiates its kernels (the instances take minutes to compile, so they are spread over
-// several units).  kind: 1 Cartesian, 0 general blocks; minw = register budget in waves per SIMD (2, 3
-// or 4), limited to those that compile without heavy spilling: fused <= 3 (2 for the generic
-// limiter), reconstruction 3-4 (3 generic); the y-face and update kernels need no limiter and are
+// several units).  kind: 1 Cartesian, 0 general blocks; minw = register budget asked for (2, 3 or 4), which
+// each launcher turns into the waves per SIMD of its instances, those that compile without heavy
+// spilling: fused and paired 2-3 (2 generic), strip reconstruction 2-3 (2 generic), row-major
+// reconstruction 3-4 (4 with HLLL, 3 generic); the y-face and update kernels need no limiter and are
 // built once.
 struct k_stage_tag {
     static void launch(const phx_plan* P, int kind, int minw, dim3 g, hipStream_t st, const StageArgs& A);

@@ -20,13 +20,16 @@ void k_recon_x_lin_tag::launch(const phx_plan* P, int kind, int minw, dim3 g, hi
     dispatch<k_recon_x_lin_go>(P, kind, minw, g, st, A);
 }
 
-// one launch of the reconstruction kernel of variant 7 over the merged list of both geometry kinds
+// One launch of the reconstruction kernel of variant 7 over the merged list of both geometry kinds.  Its
+// instances hold both kinds' paths: at 4 waves per SIMD the HLLL one spills 57 registers (6 in the
+// instances of one kind), so it takes 3 where those take 4 (ramps, us per stage at 3 and 4 waves:
+// 4 x 200^2 cells 38.5 and 40.5, 4 x 300^2 57.5 and 60.4, 5 x 500^2 168.9 and 189.7).
 void launch_recon_x_lin_mixed(const phx_plan* P, StageArgs A, hipStream_t st) {
     A.items = P->ditems_m[2];
     A.nitems = P->n_m[2];
     const dim3 g(P->grid_m[2] + A.fold_blocks), b(WAVE);
     const bool gen = generic_instance(P), roe = P->flux == PHX_FLUX_ROE;
-    const bool w4 = !gen && P->waves_per_simd >= 4;  // the register budgets the per-kind launches use
+    const bool w4 = !gen && P->waves_per_simd >= 4;
 #define PHX_RX(F, M, G) hipLaunchKernelGGL((k_recon_x_lin<2, F, M, G>), g, b, 0, st, A)
     if (gen) { if (roe) PHX_RX(0, 3, true); else PHX_RX(1, 3, true); }
     else if (w4) { if (roe) PHX_RX(0, 4, false); else PHX_RX(1, 4, false); }

@@ -29,7 +29,7 @@ void launch_recon_x_mixed(const phx_plan* P, StageArgs A, hipStream_t st) {
     A.nitems = P->n_m[0];
     const dim3 g(P->grid_m[0] + A.fold_blocks), b(WAVE);
     const bool gen = generic_instance(P), roe = P->flux == PHX_FLUX_ROE;
-    const bool w4 = !gen && P->waves_per_simd >= 4;  // the register budgets the per-kind launches use
+    const bool w4 = !gen && P->waves_per_simd >= 4;  // recon_waves: the budgets of the launches per kind
 #define PHX_RX(F, M, G) hipLaunchKernelGGL((k_recon_x<2, F, M, G>), g, b, 0, st, A)
     if (gen) { if (roe) PHX_RX(0, 2, true); else PHX_RX(1, 2, true); }
     else if (w4) { if (roe) PHX_RX(0, 3, false); else PHX_RX(1, 3, false); }
