@@ -68,9 +68,9 @@ def build_library(verbose: bool = False, extra_flags=None) -> Path:
 
 
 def build_test_library(verbose: bool = False) -> Path:
-    """Compile the tests' native libraries (tests/native/lib{device,inrange}_numerics.so)."""
+    """Compile the tests' native libraries (tests/native/lib{device,inrange,guards}_numerics.so)."""
     native = PKG.parent / "tests" / "native"
-    for name in ("device_numerics", "inrange_numerics"):
+    for name in ("device_numerics", "inrange_numerics", "guards_numerics"):
         out = native / f"lib{name}.so"
         tmp = out.with_suffix(".so.tmp")
         cmd = [HIPCC, *HIP_FLAGS, "-shared", f"-I{INCLUDE}", str(native / f"{name}.hip"), "-o", str(tmp)]

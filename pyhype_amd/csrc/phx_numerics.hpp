@@ -75,12 +75,14 @@ __host__ __device__ inline Q4 q4zero() {
 }
 
 // IEEE division by a divisor whose magnitude, and that of the numerators, is known to be moderate.  The
-// compiler's sequence for n / d scales d and n where their exponents are extreme (v_div_scale), refines
-// v_rcp_f64 by two Newton steps, forms q = n*y, the remainder r = n - d*q and q + r*y (v_div_fmas,
-// which undoes the scaling), and replaces the result where an operand is zero, infinite or NaN or the
-// quotient is not a normal number (v_div_fixup).  For 2^-700 < |d| < 2^700 and |n / d| in
-// [2^-760, 2^760] with |n| > 2^-900 the scalings and that replacement are identities, so the
-// refinement alone gives the same bits: 8 instead of 11 instructions, no dependence on VCC between
+// compiler's sequence for n / d scales d and n where their exponents are extreme (v_div_scale: a divisor or
+// quotient that is not normal, a divisor whose reciprocal is not, quotients from 2^768, numerators below
+// 2^-969), refines v_rcp_f64 by two Newton steps, forms q = n*y, the remainder r = n - d*q and q + r*y
+// (v_div_fmas, which undoes the scaling), and replaces the result where an operand is zero, infinite or
+// NaN or the quotient is not a normal number (v_div_fixup).  For 2^-1000 <= |d| <= 2^1000, |n| >= 2^-900 and
+// |n / d| in [2^-760, 2^760] the scalings and that replacement are identities, the reciprocal and its
+// refinement stay normal, and so does the remainder, a multiple of 2^-106 |n|; so the refinement
+// alone gives the same bits: 8 instead of 11 instructions, no dependence on VCC between
 // two divisions, and one reciprocal for all numerators of a divisor (3 instructions each, 2 for 1/d).
 // A numerator of +-0 gives the zero of the right sign for d > 0 (the remainder is formed as d*q - n
 // so that -0 survives); for d < 0 the sign of a zero quotient is not defined.
@@ -995,7 +997,8 @@ __host__ __device__ inline T vmax(T a, T b) { return fmax(a, b); }
 template <class T>
 __host__ __device__ inline T vmin(T a, T b) { return fmin(a, b); }
 
-// Venkatakrishnan's value for a slope s >= 0 of at most 2^495: both divisions' operands in range
+// Venkatakrishnan's value for a slope s that is 0 or in [2^-680, 2^496]: the divisor lies in [2, 2^993] and the
+// quotient in [2^-680, 2], in Recip's range
 __host__ __device__ inline double venkat_in_range(double s) {
     const double s2 = s * s;
     return Recip(s2 + s + 2.0).div(s2 + 2.0 * s);
