@@ -81,25 +81,37 @@ def validate_config(config) -> List[List[float]]:
 
 # Launch shape of a workload without a tuned one (us per RK stage measured on an MI355X, 256 CUs, smooth
 # flow, the alternatives beside it):
-#  * The shared-halo stage (variant 2) while its workgroups, one per CU, fit about one and a half rounds
-#    of the chip: with one row each up to 256 workgroups (64^2: 11.0 against 14.6 with the split
-#    stage and 25.7 fused; 8 x 32^2: 11.1 against 15.9), with two rows up to 384 (128^2, 192 of them:
-#    11.7 against 14.9; six 93 x 61 HLLL blocks, 372: 25.5 against 32.4).  At 500 it falls behind (5 x
-#    100^2 HLLL: 26.3 against 22.5; 4 x 70^2 of both geometry kinds, 560 and 280: 26.8 and 21.8 against
-#    21.0).
+#  * The shared-halo stage (variant 2) while its workgroups, one per CU, fit the chip: with one row each up to
+#    256 workgroups (120^2, 240 of them: 9.4 against 13.4 with the split stage and 26.7 fused; 64^2: 11.0,
+#    14.6 and 25.7), with two rows beyond (160^2, 240: 10.7 against 13.8; 60 x 512, 256: 10.9 against 13.9; HLLL
+#    14.2 against 19.8).  Between 257 and 384 workgroups of two rows, a second round, neither stage is the
+#    faster one throughout.  A list whose length is no multiple of 8 gives some workgroup two items (an XCD's
+#    share of the items and of the workgroups are rounded differently: 60 x 500, 250 workgroups, takes 17.3
+#    where 256 take 10.9), which costs the split stage most, with its short items: six 93 x 61 HLLL quads,
+#    372, 24.1 against 30.7; 60 x 700, 350, 18.6 against 19.8 (HLLL 23.2 and 26.0); 180^2, 270, 17.5 against
+#    20.0.  Where its lists do divide by 8 the split stage takes 15 to 23 % less with Roe and 2 to 11 % less
+#    with HLLL (60 x 768, 384: 18.8 against 14.6, HLLL 23.6 and 20.9; 5 x 64^2, 320: 18.3 against 14.1, 22.2
+#    and 20.4; 4 x 70^2, 280: 18.8 against 16.0, 22.2 and 21.8).  The fused stage takes 26 to 45 in all of these.
+#    At 500 the shared-halo stage is behind in any case (5 x 100^2 HLLL: 26.3 against 22.5).
 #  * The split stage with one y-face per wave up to the size where the states that pass between its
 #    kernels no longer stay in the caches: strips (variant 6) while a Cartesian mesh has fewer than 10^5
 #    cells (256^2: 18.2 against 20.4), row-major (variant 7) beyond (400^2: 26.6 against 27.4;
 #    8 x 150^2: 29.5 against 33.8), up to 10^6 cells with Roe (1.1 x 10^6: 98 against 96 fused;
 #    2.25 x 10^6: 220 against 167) and 2.5 x 10^6 with HLLL, whose fused kernel is bound by its
 #    registers (1.1 x 10^6: 120 against 136; 2.8 x 10^6: 319 against 326).
-#    From 2.5 x 10^5 cells the work lists are dealt to the XCDs in chunks of 64 items, so that the faces
-#    of neighbouring rows meet in one L2 (8 x 10^5: 94.1 against 99.6).
+#    From 2.5 x 10^5 cells the work lists are dealt to the XCDs in chunks of 64 items, which evens out flows
+#    that cost more in one part of the mesh (a shock, HLLL: 5 x 240^2 38.8 -> 35.1, 5 x 450^2 82.7 -> 75.1,
+#    4 x 640 x 240 64.9 -> 62.5; a blast or waves everywhere: between 4 % less and 3 % more from 2.9 x 10^5 to
+#    10^6 cells).  Smaller meshes have too few chunks to spread evenly over 8 XCDs (400^2 has 41: 22.1 -> 25.9;
+#    330^2 19.3 -> 21.6), or happen to have a good number (8 x 150^2, 46: 27.6 -> 27.2, shock 34.7 -> 33.5).
 #  * The fused stage beyond, with items of 8 rows or more (1.1 x 10^6 cells: 4 rows 111.9, 8 rows 96.2;
 #    2.4 x 10^6: 4 rows 221.6, 10 rows 201.0).
-#  * More than one Gauss point per face: strips, one row per item (two take 110 to 2 % longer from 40^2 to
-#    800 x 600 cells), with 1, 2 or 3 rows of the update (two points, 100^2: 18.8, 23.0, 23.0; 200 x 120: 22.3,
-#    20.8, 21.7; 800 x 600: 99.8, 93.4, 91.0).
+#  * More than one Gauss point per face: strips, one row per item (two take 33 to 180 % longer up to 1.2 x 10^5
+#    cells, 0 to 5 % from 1.6 x 10^5), with 1, 2 or 3 rows of the update.  Two points with Roe and
+#    Venkatakrishnan's limiter, with 1, 2, 3 rows: 100^2 23.9, 27.7, 27.8; 200 x 120 27.3, 25.7, 27.0; 400^2 59.1, 58.2, 56.0; 800 x 600 133, 128, 126.  HLLL, three
+#    points and general blocks order the same way (100^2 HLLL 36.5, 42.5, 42.3; three points 30.1, 35.0, 35.8;
+#    800 x 600 general HLLL with three 251, 235, 230); of 13 sizes only 4 x 61 x 55, whose list divides
+#    unevenly, is more than 4 % from the best of the three (31.6, 28.1, 32.6).
 SHARED_ITEMS = (256, 384)          # workgroups of the shared-halo stage with 1 and 2 rows
 STRIP_CELLS = 100_000
 DEALT_CELLS = 250_000
