@@ -91,7 +91,9 @@ def validate_config(config) -> List[List[float]]:
 #    372, 24.1 against 30.7; 60 x 700, 350, 18.6 against 19.8 (HLLL 23.2 and 26.0); 180^2, 270, 17.5 against
 #    20.0.  Where its lists do divide by 8 the split stage takes 15 to 23 % less with Roe and 2 to 11 % less
 #    with HLLL (60 x 768, 384: 18.8 against 14.6, HLLL 23.6 and 20.9; 5 x 64^2, 320: 18.3 against 14.1, 22.2
-#    and 20.4; 4 x 70^2, 280: 18.8 against 16.0, 22.2 and 21.8).  The fused stage takes 26 to 45 in all of these.
+#    and 20.4; 4 x 70^2, 280: 18.8 against 16.0, 22.2 and 21.8).  The same happens below 256 where only the
+#    shared-halo stage's own count does not divide (60 x 280, 140: 17.8 against 14.4; 180 x 168, 252: 16.7
+#    against 13.8).  The fused stage takes 26 to 45 in all of these.
 #    At 500 the shared-halo stage is behind in any case (5 x 100^2 HLLL: 26.3 against 22.5).
 #  * The split stage with one y-face per wave up to the size where the states that pass between its
 #    kernels no longer stay in the caches: strips (variant 6) while a Cartesian mesh has fewer than 10^5
@@ -108,10 +110,11 @@ def validate_config(config) -> List[List[float]]:
 #    2.4 x 10^6: 4 rows 221.6, 10 rows 201.0).
 #  * More than one Gauss point per face: strips, one row per item (two take 33 to 180 % longer up to 1.2 x 10^5
 #    cells, 0 to 5 % from 1.6 x 10^5), with 1, 2 or 3 rows of the update.  Two points with Roe and
-#    Venkatakrishnan's limiter, with 1, 2, 3 rows: 100^2 23.9, 27.7, 27.8; 200 x 120 27.3, 25.7, 27.0; 400^2 59.1, 58.2, 56.0; 800 x 600 133, 128, 126.  HLLL, three
-#    points and general blocks order the same way (100^2 HLLL 36.5, 42.5, 42.3; three points 30.1, 35.0, 35.8;
-#    800 x 600 general HLLL with three 251, 235, 230); of 13 sizes only 4 x 61 x 55, whose list divides
-#    unevenly, is more than 4 % from the best of the three (31.6, 28.1, 32.6).
+#    Venkatakrishnan's limiter, with 1, 2, 3 rows: 100^2 23.9, 27.7, 27.8; 200 x 120 27.3, 25.7, 27.0; 400^2
+#    59.1, 58.2, 56.0; 800 x 600 133, 128, 126.  HLLL, three points and general blocks order the same way
+#    (100^2 HLLL 36.5, 42.5, 42.3; three points 30.1, 35.0, 35.8; 800 x 600 general HLLL with three 251, 235,
+#    230); of 13 sizes only 4 x 61 x 55, whose list divides unevenly, is more than 4 % from the best of the
+#    three (31.6, 28.1, 32.6).
 SHARED_ITEMS = (256, 384)          # workgroups of the shared-halo stage with 1 and 2 rows
 STRIP_CELLS = 100_000
 DEALT_CELLS = 250_000
